@@ -11,7 +11,7 @@
 //   res = v_div_fixup(d, b, a)      = d unless an operand or the result is
 //                                     zero, infinite, NaN or out of range
 //
-// When |a| and |b| lie in [2^-380, 2^380] (or a is zero), the scaling steps
+// When |a| and |b| lie in [2^-390, 2^390] (or a is zero), the scaling steps
 // return their operands unchanged: the exponent difference stays below 768,
 // neither operand nor the quotient is denormal, the numerator's exponent is
 // far above the near-underflow threshold and 1/b is normal.  In that case the
@@ -36,16 +36,21 @@
 
 namespace HYPE_KNS {
 
-constexpr double FDIV_HI = 0x1p380;
-constexpr double FDIV_LO = 0x1p-380;
+// high word of 2^388: a positive double is below 2^388 if and only if its
+// high word is below this one
+constexpr unsigned FDIV_TOP_WORD = (1023u + 388u) << 20;
+__device__ __forceinline__ unsigned hi_word(double x) { return (unsigned)__double2hiint(x); }
 
-// refined reciprocal of b, as in the division sequence
+// refined reciprocal of b.  One third-order step, y0 (1 + e + e^2) with
+// e = 1 - b y0, in place of the sequence's two Newton steps: three fused
+// operations instead of four.  |e| <= 2^-23 (the hardware's bound for
+// v_rcp_f64), so the step's own error is below 2^-68 and the result is the
+// rounded reciprocal up to 2^-15 of an ulp in the halfway cases, as the
+// quotient and remainder step below need it
 __device__ __forceinline__ double recip_nr(double b) {
-  double y = __builtin_amdgcn_rcp(b);
-  double e = fma(-b, y, 1.0);
-  y = fma(y, e, y);
-  e = fma(-b, y, 1.0);
-  return fma(y, e, y);
+  const double y = __builtin_amdgcn_rcp(b);
+  const double e = fma(-b, y, 1.0);
+  return fma(y, fma(e, e, e), y);
 }
 
 // a / b for b > 0 in range, given y = recip_nr(b); bitwise equal to a / b
@@ -59,12 +64,6 @@ __device__ __forceinline__ double div_y(double a, double b, double y) {
 __device__ __forceinline__ double inv_y(double b, double y) {
   const double rn = fma(b, y, -1.0);
   return fma(-rn, y, y);
-}
-
-// |x| in [2^-380, 2^380]; false for zero, NaN and infinities
-__device__ __forceinline__ bool fdiv_in_range(double x) {
-  const double a = fabs(x);
-  return a >= FDIV_LO && a <= FDIV_HI;
 }
 
 }  // namespace HYPE_KNS

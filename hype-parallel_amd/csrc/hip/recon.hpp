@@ -14,6 +14,8 @@
 #endif
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
 #include "fdiv.hpp"
 
 namespace HYPE_KNS {
@@ -86,14 +88,51 @@ struct Quad {
   static constexpr double gphy(int q, int k) { return basis_gy(volx(q), voly(q), k); }
 };
 
-// sum_k s[k]*phi(k) in the reference's order, skipping exact-zero phi
-#define HYPE_BASIS_SUM(out, s, NDOF, PHI)               \
-  do {                                                  \
-    double acc_ = 0.0;                                  \
-    _Pragma("unroll") for (int k_ = 0; k_ < NDOF; ++k_) \
-      if (PHI(k_) != 0.0) acc_ = acc_ + s[k_] * PHI(k_); \
-    out = acc_;                                         \
-  } while (0)
+constexpr bool is_pow2(double x) {
+  x = x < 0.0 ? -x : x;
+  if (x == 0.0) return false;
+  while (x < 1.0) x *= 2.0;
+  while (x > 1.0) x *= 0.5;
+  return x == 1.0;
+}
+
+// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>): a loop
+// whose index is a constant expression in its body
+template <class F, int... I>
+__device__ __forceinline__ void static_for_seq(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// sum_k s[k]*phi(k) in the reference's order, skipping exact-zero phi; T::at(k)
+// is the table row.  A product with a power of two is exact, so fusing it with
+// the addition rounds once, as the separate operations do, in one instruction
+template <class T, int NDOF>
+__device__ __forceinline__ double basis_sum(const double* s) {
+  double acc = 0.0;
+  static_for<NDOF>([&](auto K) {
+    constexpr int k = decltype(K)::value;
+    constexpr double phi = T::at(k);
+    if constexpr (is_pow2(phi))
+      acc = fma(s[k], phi, acc);
+    else if constexpr (phi != 0.0)
+      acc = acc + s[k] * phi;
+  });
+  return acc;
+}
+
+// rows of the tables: node P, volume point Q and its gradients
+template <int N, int P>
+struct RowNode { static constexpr double at(int k) { return Quad<N>::phin(P, k); } };
+template <int N, int Q>
+struct RowVol { static constexpr double at(int k) { return Quad<N>::phiv(Q, k); } };
+template <int N, int Q>
+struct RowGx { static constexpr double at(int k) { return Quad<N>::gphx(Q, k); } };
+template <int N, int Q>
+struct RowGy { static constexpr double at(int k) { return Quad<N>::gphy(Q, k); } };
 
 // reconstruction.c:106-117
 __device__ __forceinline__ double minmod(double a, double b) {
@@ -107,92 +146,95 @@ __device__ __forceinline__ double pow4(double a) {  // reconstruction.c:123-127
   return a2 * a2;
 }
 
+// One direction of weno3 (reconstruction.c:155-187): the three candidates'
+// slopes and curvatures and their nonlinear combination.  The candidates are
+// kept doubled (S_i = 2 u_x,i, s_i = 2 u_xx,i): scaling by a power of two is
+// exact, so every sum and product is the reference's times a power of two, and
+// its products with 2 and 1/2 become the exact operand of a fused
+// multiply-add: 11 operations for the six candidate values instead of 20.  The
+// smoothness terms are then 4 times, their fourth powers 256 times the
+// reference's, which cancels in the weights; dividing by twice the weights' sum
+// undoes the doubling.  T3 = 3 u_0.  top: running maximum of the high words of
+// the divisors.
+__device__ __forceinline__ void weno3_dir(double m2, double m1, double u0, double p1, double p2, double T3,
+                                          double& slope, double& curv, unsigned& top) {
+  const double r13_3 = 13. / 3.;
+  const double S0 = fma(-4.0, m1, m2) + T3;
+  const double S1 = p1 - m1;
+  const double S2 = fma(4.0, p1, -T3) - p2;
+  const double s0 = fma(-2.0, m1, m2) + u0;
+  const double s1 = fma(-2.0, u0, m1) + p1;
+  const double s2 = fma(-2.0, p1, u0) + p2;
+  const double d0 = pow4(S0 * S0 + r13_3 * s0 * s0 + 4.0 * SMALL_NUM);
+  const double d1 = pow4(S1 * S1 + r13_3 * s1 * s1 + 4.0 * SMALL_NUM);
+  const double d2 = pow4(S2 * S2 + r13_3 * s2 * s2 + 4.0 * SMALL_NUM);
+  top = max(top, max(max(hi_word(d0), hi_word(d1)), hi_word(d2)));
+  double w0 = inv_y(d0, recip_nr(d0));
+  double w1 = div_y(100.0, d1, recip_nr(d1));  // the central cell's linear weight
+  double w2 = inv_y(d2, recip_nr(d2));
+  const double total = w0 + w1 + w2;
+  const double total2 = total + total;
+  const double yt = recip_nr(total2);
+  w0 = div_y(w0, total2, yt);
+  w1 = div_y(w1, total2, yt);
+  w2 = div_y(w2, total2, yt);
+  slope = w0 * S0 + w1 * S1 + w2 * S2;
+  curv = w0 * s0 + w1 * s1 + w2 * s2;
+}
+
 // weno3 with every division done by fdiv.hpp's shared-reciprocal sequence.
 // Same expressions and operation order as the reference weno3
-// (reconstruction.c:144-221), so the coefficients are bitwise those of the
-// IEEE-division version whenever all divisors are in range; returns false
-// otherwise (the caller then recomputes with plain division).  The divisors
-// are pow4(IS + 1e-12) >= 1e-48 and the weight sums; a group is in range when
-// the sum of its pow4 terms is at most 2^380 (then every weight and sum lies
-// in [2^-380, 2^380]).
+// (reconstruction.c:144-221) up to exact scalings by powers of two, so the
+// coefficients are bitwise those of the IEEE-division version whenever all
+// divisors are in range; returns false otherwise (the caller then recomputes
+// with plain division).  The divisors are the pow4 terms, >= 1e-48, and the
+// weight sums; all are in range when every pow4 term is below 2^388.  The
+// terms are positive (or NaN, whose high word is larger still), so their high
+// words compare as they do.
+//
+// The stage kernel is bound by FP64 issue and this is half of a row's
+// instructions: 248 per component (288 with the unscaled candidates, two
+// Newton steps per reciprocal and FP64 range checks).  Measured over an SSP-RK
+// solve: Kapila 1024x512 4802 -> 4503 us per 10 steps, Baer-Nunziato 2048x1024
+// 9191 -> 8647 us per 3, Euler 256x256 2007 -> 1934 us per 20.
 __device__ __forceinline__ bool weno3_fast(const double* U_x, const double* U_y, const double* U_xy,
                                            double* coeffs) {
-  const double central_cell_wt = 100.0;
-  const double r13_3 = 13. / 3.;
-  double u_0 = U_xy[0];
-  double u_ip1 = U_x[3], u_jp1 = U_y[3], u_ip1jp1 = U_xy[1];
-  double u_im1 = U_x[1], u_jm1 = U_y[1], u_ip1jm1 = U_xy[2];
-  double u_ip2 = U_x[4], u_jp2 = U_y[4], u_im1jp1 = U_xy[3];
-  double u_im2 = U_x[0], u_jm2 = U_y[0], u_im1jm1 = U_xy[4];
-  double ux0, ux1, ux2, uxx0, uxx1, uxx2, d0, d1, d2, d3, w0, w1, w2, w3, total, yt, temp;
-  bool ok;
-
-  ux0 = -2.0 * u_im1 + 0.5 * u_im2 + 1.5 * u_0;
-  uxx0 = 0.5 * (u_im2 - 2.0 * u_im1 + u_0);
-  ux1 = 0.5 * (u_ip1 - u_im1);
-  uxx1 = 0.5 * (u_im1 - 2.0 * u_0 + u_ip1);
-  ux2 = -1.5 * u_0 + 2.0 * u_ip1 - 0.5 * u_ip2;
-  uxx2 = 0.5 * (u_0 - 2.0 * u_ip1 + u_ip2);
-  d0 = pow4(ux0 * ux0 + r13_3 * uxx0 * uxx0 + SMALL_NUM);
-  d1 = pow4(ux1 * ux1 + r13_3 * uxx1 * uxx1 + SMALL_NUM);
-  d2 = pow4(ux2 * ux2 + r13_3 * uxx2 * uxx2 + SMALL_NUM);
-  ok = (d0 + d1 + d2) <= FDIV_HI;
-  w0 = inv_y(d0, recip_nr(d0));
-  w1 = div_y(central_cell_wt, d1, recip_nr(d1));
-  w2 = inv_y(d2, recip_nr(d2));
-  total = w0 + w1 + w2;
-  yt = recip_nr(total);
-  w0 = div_y(w0, total, yt);
-  w1 = div_y(w1, total, yt);
-  w2 = div_y(w2, total, yt);
+  const double u_0 = U_xy[0];
+  const double T3 = 3.0 * u_0;
+  unsigned top = 0;
+  double c1, c2, c3, c4;
+  weno3_dir(U_x[0], U_x[1], u_0, U_x[3], U_x[4], T3, c1, c3, top);
+  weno3_dir(U_y[0], U_y[1], u_0, U_y[3], U_y[4], T3, c2, c4, top);
   coeffs[0] = u_0;
-  coeffs[1] = w0 * ux0 + w1 * ux1 + w2 * ux2;
-  coeffs[3] = w0 * uxx0 + w1 * uxx1 + w2 * uxx2;
+  coeffs[1] = c1;
+  coeffs[2] = c2;
+  coeffs[3] = c3;
+  coeffs[4] = c4;
 
-  ux0 = -2.0 * u_jm1 + 0.5 * u_jm2 + 1.5 * u_0;
-  uxx0 = 0.5 * (u_jm2 - 2.0 * u_jm1 + u_0);
-  ux1 = 0.5 * (u_jp1 - u_jm1);
-  uxx1 = 0.5 * (u_jm1 - 2.0 * u_0 + u_jp1);
-  ux2 = -1.5 * u_0 + 2.0 * u_jp1 - 0.5 * u_jp2;
-  uxx2 = 0.5 * (u_0 - 2.0 * u_jp1 + u_jp2);
-  d0 = pow4(ux0 * ux0 + r13_3 * uxx0 * uxx0 + SMALL_NUM);
-  d1 = pow4(ux1 * ux1 + r13_3 * uxx1 * uxx1 + SMALL_NUM);
-  d2 = pow4(ux2 * ux2 + r13_3 * uxx2 * uxx2 + SMALL_NUM);
-  ok = ok && (d0 + d1 + d2) <= FDIV_HI;
-  w0 = inv_y(d0, recip_nr(d0));
-  w1 = div_y(central_cell_wt, d1, recip_nr(d1));
-  w2 = inv_y(d2, recip_nr(d2));
-  total = w0 + w1 + w2;
-  yt = recip_nr(total);
-  w0 = div_y(w0, total, yt);
-  w1 = div_y(w1, total, yt);
-  w2 = div_y(w2, total, yt);
-  coeffs[2] = w0 * ux0 + w1 * ux1 + w2 * ux2;
-  coeffs[4] = w0 * uxx0 + w1 * uxx1 + w2 * uxx2;
-
-  double c1 = coeffs[1], c2 = coeffs[2], c3 = coeffs[3], c4 = coeffs[4];
-  double uxy0 = u_ip1jp1 - u_0 - c1 - c2 - c3 - c4;
-  double uxy1 = -u_ip1jm1 + u_0 + c1 - c2 + c3 + c4;
-  double uxy2 = -u_im1jp1 + u_0 - c1 + c2 + c3 + c4;
-  double uxy3 = u_im1jm1 - u_0 + c1 + c2 - c3 - c4;
-  temp = 4.0 * (c3 * c3 + c4 * c4);
-  d0 = pow4(temp + uxy0 * uxy0 + SMALL_NUM);
-  d1 = pow4(temp + uxy1 * uxy1 + SMALL_NUM);
-  d2 = pow4(temp + uxy2 * uxy2 + SMALL_NUM);
-  d3 = pow4(temp + uxy3 * uxy3 + SMALL_NUM);
-  ok = ok && (d0 + d1 + d2 + d3) <= FDIV_HI;
-  w0 = inv_y(d0, recip_nr(d0));
-  w1 = inv_y(d1, recip_nr(d1));
-  w2 = inv_y(d2, recip_nr(d2));
-  w3 = inv_y(d3, recip_nr(d3));
-  total = w0 + w1 + w2 + w3;
-  yt = recip_nr(total);
+  // U_xy: u_0, u_ip1jp1, u_ip1jm1, u_im1jp1, u_im1jm1
+  const double uxy0 = U_xy[1] - u_0 - c1 - c2 - c3 - c4;
+  const double uxy1 = -U_xy[2] + u_0 + c1 - c2 + c3 + c4;
+  const double uxy2 = -U_xy[3] + u_0 - c1 + c2 + c3 + c4;
+  const double uxy3 = U_xy[4] - u_0 + c1 + c2 - c3 - c4;
+  const double t = c3 * c3 + c4 * c4;
+  const double d0 = pow4(fma(4.0, t, uxy0 * uxy0) + SMALL_NUM);
+  const double d1 = pow4(fma(4.0, t, uxy1 * uxy1) + SMALL_NUM);
+  const double d2 = pow4(fma(4.0, t, uxy2 * uxy2) + SMALL_NUM);
+  const double d3 = pow4(fma(4.0, t, uxy3 * uxy3) + SMALL_NUM);
+  top = max(top, max(max(hi_word(d0), hi_word(d1)), hi_word(d2)));
+  top = max(top, hi_word(d3));
+  double w0 = inv_y(d0, recip_nr(d0));
+  double w1 = inv_y(d1, recip_nr(d1));
+  double w2 = inv_y(d2, recip_nr(d2));
+  double w3 = inv_y(d3, recip_nr(d3));
+  const double total = w0 + w1 + w2 + w3;
+  const double yt = recip_nr(total);
   w0 = div_y(w0, total, yt);
   w1 = div_y(w1, total, yt);
   w2 = div_y(w2, total, yt);
   w3 = div_y(w3, total, yt);
   coeffs[5] = w0 * uxy0 + w1 * uxy1 + w2 * uxy2 + w3 * uxy3;
-  return ok;
+  return top < FDIV_TOP_WORD;
 }
 
 // reconstruction.c:223-357: CWENO with one fourth-degree central candidate

@@ -227,33 +227,23 @@ struct Tile {
   static_assert(XST <= XCH, "the lower wave's staging must fit its exchange area");
   static constexpr int LDS = WAVES * WIN + (PAIR ? 2 * XCH + DEFER : 0) + WAVES * OST + (COMBINE ? 1 : 0) + XST;
 
-  // value of component c at node/face point p from its modal coefficients
+  // values of all components at the nodes, which are the face points
   // (rhs_function_prim.c:382-388, 425-440)
-  __device__ static __forceinline__ double at_node(const double (&co)[NV][NDOF], int c, int p) {
-    double v;
-#define PHIN(k) Qd::phin(p, k)
-    HYPE_BASIS_SUM(v, co[c], NDOF, PHIN);
-#undef PHIN
-    return v;
+  __device__ static __forceinline__ void at_nodes(const double (&co)[NV][NDOF], double (&fv)[NNODE][NV]) {
+    static_for<NNODE>([&](auto P) {
+#pragma unroll
+      for (int c = 0; c < NV; ++c) fv[P][c] = basis_sum<RowNode<N, P>, NDOF>(co[c]);
+    });
   }
   // value and scaled gradient at volume point q (rhs_function_prim.c:442-455)
-  __device__ static __forceinline__ void at_vol(const double (&co)[NV][NDOF], int q, double r1_h, double* V,
-                                                double* gx, double* gy) {
+  template <int q>
+  __device__ static __forceinline__ void at_vol(const double (&co)[NV][NDOF], double r1_h, double* V, double* gx,
+                                                double* gy) {
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
-      double a, b, d;
-#define PHIV(k) Qd::phiv(q, k)
-#define GPX(k) Qd::gphx(q, k)
-#define GPY(k) Qd::gphy(q, k)
-      HYPE_BASIS_SUM(a, co[c], NDOF, PHIV);
-      HYPE_BASIS_SUM(b, co[c], NDOF, GPX);
-      HYPE_BASIS_SUM(d, co[c], NDOF, GPY);
-#undef PHIV
-#undef GPX
-#undef GPY
-      V[c] = a;
-      gx[c] = r1_h * b;
-      gy[c] = r1_h * d;
+      V[c] = basis_sum<RowVol<N, q>, NDOF>(co[c]);
+      gx[c] = r1_h * basis_sum<RowGx<N, q>, NDOF>(co[c]);
+      gy[c] = r1_h * basis_sum<RowGy<N, q>, NDOF>(co[c]);
     }
   }
 
@@ -678,10 +668,7 @@ struct Tile {
       // values at the nodes, which are also the face quadrature points
       // (rhs_function_prim.c:382-388, 425-440; the same points, hype.c:207-229)
       double fv[NNODE][NV];
-#pragma unroll
-      for (int p = 0; p < NNODE; ++p)
-#pragma unroll
-        for (int c = 0; c < NV; ++c) fv[p][c] = at_node(co, c, p);
+      at_nodes(co, fv);
       // admissibility at the nodes (rhs_function_prim.c:393-404); with
       // ACACHE the check's a_sq at each node goes on to the flux there
       double an[ACACHE ? NNODE : 1];
@@ -705,10 +692,7 @@ struct Tile {
 #pragma unroll
           for (int k = 3; k < NDOF; ++k) co[c][k] = 0.0;
         }
-#pragma unroll
-        for (int p = 0; p < NNODE; ++p)
-#pragma unroll
-          for (int c = 0; c < NV; ++c) fv[p][c] = at_node(co, c, p);
+        at_nodes(co, fv);
         if constexpr (ACACHE) {
 #pragma unroll
           for (int p = 0; p < NNODE; ++p) an[p] = -1.0;  // new values: the flux computes a_sq itself
@@ -739,15 +723,14 @@ struct Tile {
       for (int c = 0; c < NV; ++c) ncp[c] = 0.0;
       if constexpr (S::HAS_NCP) {
         if (mode != HYPE_MODE_PRIME && ownedRow) {
-#pragma unroll
-          for (int q = 0; q < NGV; ++q) {
+          static_for<NGV>([&](auto q) {
             double V[NV], gx[NV], gy[NV], B[NV];
-            at_vol(co, q, r1_h, V, gx, gy);
+            at_vol<q>(co, r1_h, V, gx, gy);
             S::template vol_ncp<PRIM>(eos, V, gx, gy, B);
 #pragma unroll
             for (int c = 0; c < NV; ++c)
               if (S::DNZ[c]) ncp[c] = ncp[c] + -WV * B[c];
-          }
+          });
         }
       }
 
