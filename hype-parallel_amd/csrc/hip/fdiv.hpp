@@ -66,4 +66,34 @@ __device__ __forceinline__ double inv_y(double b, double y) {
   return fma(-rn, y, y);
 }
 
+// a / b for a b that is the same for every cell, given y = recip_nr(b): the
+// quotient step and the sequence's fixup, 4 instructions instead of 11.  The
+// fixup handles zeros, infinities and NaN.  b is a product of (gamma - 1)
+// factors, so 0 or at least 2^-105 in magnitude; a is a sum of products of
+// pressures, zero or far above 2^-960, where the remainder would no longer be
+// exact.
+__device__ __forceinline__ double div_const(double a, double b, double y) {
+  return __builtin_amdgcn_div_fixup(div_y(a, b, y), b, a);
+}
+
+// sqrt(x) for x >= 2^-767, and for zero, infinity, NaN and negative x: one
+// coupled Newton step for the root g and its half reciprocal h (error below
+// 2^-44), then two corrections with the exact remainder x - g^2, the second of
+// which rounds correctly.  Without the rescaling of tiny arguments it takes 13
+// instructions instead of 18.  Arguments are squared sound speeds, at least
+// 1e-12 or already reported as inadmissible.
+__device__ __forceinline__ double sqrt_adm(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y;
+  double h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  double d = fma(-g, g, x);
+  g = fma(d, h, g);
+  d = fma(-g, g, x);
+  g = fma(d, h, g);
+  return __builtin_amdgcn_class(x, 0x260) ? x : g;  // +inf, +0 and -0
+}
+
 }  // namespace HYPE_KNS

@@ -109,14 +109,15 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 // sum_k s[k]*phi(k) in the reference's order, skipping exact-zero phi; T::at(k)
 // is the table row.  A product with a power of two is exact, so fusing it with
-// the addition rounds once, as the separate operations do, in one instruction
-template <class T, int NDOF>
+// the addition rounds once, as the separate operations do, in one instruction.
+// TINY: the component may hold subnormal values (S::TINY), whose halves round
+template <class T, int NDOF, bool TINY>
 __device__ __forceinline__ double basis_sum(const double* s) {
   double acc = 0.0;
   static_for<NDOF>([&](auto K) {
     constexpr int k = decltype(K)::value;
     constexpr double phi = T::at(k);
-    if constexpr (is_pow2(phi))
+    if constexpr (is_pow2(phi) && (!TINY || phi >= 1.0))
       acc = fma(s[k], phi, acc);
     else if constexpr (phi != 0.0)
       acc = acc + s[k] * phi;
@@ -154,32 +155,44 @@ __device__ __forceinline__ double pow4(double a) {  // reconstruction.c:123-127
 // multiply-add: 11 operations for the six candidate values instead of 20.  The
 // smoothness terms are then 4 times, their fourth powers 256 times the
 // reference's, which cancels in the weights; dividing by twice the weights' sum
-// undoes the doubling.  T3 = 3 u_0.  top: running maximum of the high words of
+// undoes the doubling.
+// TINY: the component may hold subnormal values (S::TINY), whose products with
+// 1/2 round; the candidates then keep the reference's halves (17 operations).
+// The smoothness terms may still use the doubled curvatures: below 1e-28 they
+// vanish beside the 1e-12 they are added to.
+// h0 = 3/2 u_0 (TINY), else 3 u_0.  top: running maximum of the high words of
 // the divisors.
-__device__ __forceinline__ void weno3_dir(double m2, double m1, double u0, double p1, double p2, double T3,
+template <bool TINY>
+__device__ __forceinline__ void weno3_dir(double m2, double m1, double u0, double p1, double p2, double h0,
                                           double& slope, double& curv, unsigned& top) {
   const double r13_3 = 13. / 3.;
-  const double S0 = fma(-4.0, m1, m2) + T3;
-  const double S1 = p1 - m1;
-  const double S2 = fma(4.0, p1, -T3) - p2;
   const double s0 = fma(-2.0, m1, m2) + u0;
   const double s1 = fma(-2.0, u0, m1) + p1;
   const double s2 = fma(-2.0, p1, u0) + p2;
-  const double d0 = pow4(S0 * S0 + r13_3 * s0 * s0 + 4.0 * SMALL_NUM);
-  const double d1 = pow4(S1 * S1 + r13_3 * s1 * s1 + 4.0 * SMALL_NUM);
-  const double d2 = pow4(S2 * S2 + r13_3 * s2 * s2 + 4.0 * SMALL_NUM);
+  const double S0 = TINY ? fma(-2.0, m1, 0.5 * m2) + h0 : fma(-4.0, m1, m2) + h0;
+  const double S1 = TINY ? 0.5 * (p1 - m1) : p1 - m1;
+  const double S2 = TINY ? fma(2.0, p1, -h0) - 0.5 * p2 : fma(4.0, p1, -h0) - p2;
+  // TINY: S^2 + (r s) s / 4 + eps, else 4 times that
+  const double is0 = r13_3 * s0 * s0, is1 = r13_3 * s1 * s1, is2 = r13_3 * s2 * s2;
+  const double eps = TINY ? SMALL_NUM : 4.0 * SMALL_NUM;
+  const double d0 = pow4((TINY ? fma(0.25, is0, S0 * S0) : S0 * S0 + is0) + eps);
+  const double d1 = pow4((TINY ? fma(0.25, is1, S1 * S1) : S1 * S1 + is1) + eps);
+  const double d2 = pow4((TINY ? fma(0.25, is2, S2 * S2) : S2 * S2 + is2) + eps);
   top = max(top, max(max(hi_word(d0), hi_word(d1)), hi_word(d2)));
   double w0 = inv_y(d0, recip_nr(d0));
   double w1 = div_y(100.0, d1, recip_nr(d1));  // the central cell's linear weight
   double w2 = inv_y(d2, recip_nr(d2));
   const double total = w0 + w1 + w2;
-  const double total2 = total + total;
-  const double yt = recip_nr(total2);
-  w0 = div_y(w0, total2, yt);
-  w1 = div_y(w1, total2, yt);
-  w2 = div_y(w2, total2, yt);
+  const double sum = TINY ? total : total + total;
+  const double yt = recip_nr(sum);
+  w0 = div_y(w0, sum, yt);
+  w1 = div_y(w1, sum, yt);
+  w2 = div_y(w2, sum, yt);
   slope = w0 * S0 + w1 * S1 + w2 * S2;
-  curv = w0 * s0 + w1 * s1 + w2 * s2;
+  if constexpr (TINY)
+    curv = w0 * (0.5 * s0) + w1 * (0.5 * s1) + w2 * (0.5 * s2);
+  else
+    curv = w0 * s0 + w1 * s1 + w2 * s2;
 }
 
 // weno3 with every division done by fdiv.hpp's shared-reciprocal sequence.
@@ -193,18 +206,19 @@ __device__ __forceinline__ void weno3_dir(double m2, double m1, double u0, doubl
 // words compare as they do.
 //
 // The stage kernel is bound by FP64 issue and this is half of a row's
-// instructions: 248 per component (288 with the unscaled candidates, two
-// Newton steps per reciprocal and FP64 range checks).  Measured over an SSP-RK
+// instructions: 248 per component, 258 where it may be subnormal (288 with the
+// unscaled candidates, two Newton steps per reciprocal and FP64 range checks).  Measured over an SSP-RK
 // solve: Kapila 1024x512 4802 -> 4503 us per 10 steps, Baer-Nunziato 2048x1024
 // 9191 -> 8647 us per 3, Euler 256x256 2007 -> 1934 us per 20.
+template <bool TINY>
 __device__ __forceinline__ bool weno3_fast(const double* U_x, const double* U_y, const double* U_xy,
                                            double* coeffs) {
   const double u_0 = U_xy[0];
-  const double T3 = 3.0 * u_0;
+  const double h0 = (TINY ? 1.5 : 3.0) * u_0;
   unsigned top = 0;
   double c1, c2, c3, c4;
-  weno3_dir(U_x[0], U_x[1], u_0, U_x[3], U_x[4], T3, c1, c3, top);
-  weno3_dir(U_y[0], U_y[1], u_0, U_y[3], U_y[4], T3, c2, c4, top);
+  weno3_dir<TINY>(U_x[0], U_x[1], u_0, U_x[3], U_x[4], h0, c1, c3, top);
+  weno3_dir<TINY>(U_y[0], U_y[1], u_0, U_y[3], U_y[4], h0, c2, c4, top);
   coeffs[0] = u_0;
   coeffs[1] = c1;
   coeffs[2] = c2;
@@ -330,7 +344,7 @@ __device__ __forceinline__ void weno4(const double* U_x, const double* U_y, cons
 // Stencil of one component: x[0..4] = u(i-2..i+2, j), y[0..4] = u(i, j-2..j+2),
 // d[0..4] = u(i,j), u(i+1,j+1), u(i+1,j-1), u(i-1,j+1), u(i-1,j-1)
 // (rhs_function_prim.c:332-348).
-template <int N>
+template <int N, bool TINY>
 __device__ __forceinline__ void reconstruct(const double* U_x, const double* U_y, const double* U_xy,
                                             double* coeffs) {
   if constexpr (N == 0) {
@@ -344,7 +358,7 @@ __device__ __forceinline__ void reconstruct(const double* U_x, const double* U_y
   } else if constexpr (N == 3) {
     weno4(U_x, U_y, U_xy, coeffs);
   } else {
-    if (__builtin_expect(weno3_fast(U_x, U_y, U_xy, coeffs), 1)) return;
+    if (__builtin_expect(weno3_fast<TINY>(U_x, U_y, U_xy, coeffs), 1)) return;
     // reconstruction.c:144-221
     const double central_cell_wt = 100.0;
     const double r13_3 = 13. / 3.;

@@ -182,6 +182,12 @@ __device__ __forceinline__ double lane_from_right(double v) {
                           __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false));
 }
 
+// a value every lane computes alike, as a scalar
+__device__ __forceinline__ double uniform(double v) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
 constexpr int NSLOT = 5;
 constexpr int COLS = HYPE_WAVE + 4;
 
@@ -194,6 +200,10 @@ struct Tile {
   static constexpr int WAVES = PAIR ? 2 : 1;
   // the admissibility check's a_sq at each node goes on to the flux there
   static constexpr bool ACACHE = PRIM && S::HAS_ACACHE && N == 2;
+  // inadmissible states are looked for after each face point where the states
+  // of a face's points are too many to be kept (nine components: 191 registers
+  // spilled), else once per face, which leaves its arithmetic in one block
+  static constexpr bool CHECK_EACH = NV > 6;
   // LDS per workgroup, in doubles: one window per wave, then (paired) the
   // two exchange areas (NGF x (NV + 1) values per lane: face values and the
   // a_sq handed over with them) and the upper wave's deferred row state
@@ -227,24 +237,56 @@ struct Tile {
   static_assert(XST <= XCH, "the lower wave's staging must fit its exchange area");
   static constexpr int LDS = WAVES * WIN + (PAIR ? 2 * XCH + DEFER : 0) + WAVES * OST + (COMBINE ? 1 : 0) + XST;
 
+  // The face sums are WF * (1/2 A_q) and WF * D_q over a face's points, and the
+  // jumps enter the assembly halved: powers of two, which are taken together into
+  // one factor kf = WF / 2 on the assembled difference.  Every sum is then the
+  // reference's divided by kf, hence has its bits, unless a term is subnormal:
+  // the transverse velocity's flux and a jump with a velocity factor keep the
+  // reference's operations
+  static constexpr bool plain(int dir, int c) {
+    return S::JUMP_TINY[c] || c == (dir == 0 ? S::REFY : S::REFX)[0] || c == (dir == 0 ? S::REFY : S::REFX)[1];
+  }
+  // add point q's flux A and jump D to the sums F and E of a face
+  template <int dir>
+  __device__ static __forceinline__ void add_point(int q, const double* A, const double* D, double* F, double* E) {
+    static_for<NV>([&](auto c) {
+      const double f = plain(dir, c) ? Qd::WF * (0.5 * A[c]) : A[c];
+      F[c] = q == 0 ? f : F[c] + f;
+      if constexpr (S::DNZ[c]) {
+        const double d = plain(dir, c) ? Qd::WF * D[c] : D[c];
+        E[c] = q == 0 ? d : E[c] + d;
+      } else {
+        E[c] = 0.0;
+      }
+    });
+  }
+  // 1/h (F1 - F0 + 1/2 (E1 + E0)) of component c
+  template <int dir, int c>
+  __device__ static __forceinline__ double face_diff(double r1_h, double F1, double F0, double E1, double E0) {
+    if constexpr (!S::DNZ[c])
+      return (plain(dir, c) ? r1_h : 0.5 * Qd::WF * r1_h) * (F1 - F0);
+    else if constexpr (plain(dir, c))
+      return r1_h * (F1 - F0 + 0.5 * (E1 + E0));
+    else
+      return (0.5 * Qd::WF * r1_h) * (F1 - F0 + (E1 + E0));
+  }
+
   // values of all components at the nodes, which are the face points
   // (rhs_function_prim.c:382-388, 425-440)
   __device__ static __forceinline__ void at_nodes(const double (&co)[NV][NDOF], double (&fv)[NNODE][NV]) {
     static_for<NNODE>([&](auto P) {
-#pragma unroll
-      for (int c = 0; c < NV; ++c) fv[P][c] = basis_sum<RowNode<N, P>, NDOF>(co[c]);
+      static_for<NV>([&](auto c) { fv[P][c] = basis_sum<RowNode<N, P>, NDOF, S::TINY[c]>(co[c]); });
     });
   }
   // value and scaled gradient at volume point q (rhs_function_prim.c:442-455)
   template <int q>
   __device__ static __forceinline__ void at_vol(const double (&co)[NV][NDOF], double r1_h, double* V, double* gx,
                                                 double* gy) {
-#pragma unroll
-    for (int c = 0; c < NV; ++c) {
-      V[c] = basis_sum<RowVol<N, q>, NDOF>(co[c]);
-      gx[c] = r1_h * basis_sum<RowGx<N, q>, NDOF>(co[c]);
-      gy[c] = r1_h * basis_sum<RowGy<N, q>, NDOF>(co[c]);
-    }
+    static_for<NV>([&](auto c) {
+      V[c] = basis_sum<RowVol<N, q>, NDOF, S::TINY[c]>(co[c]);
+      gx[c] = r1_h * basis_sum<RowGx<N, q>, NDOF, S::TINY[c]>(co[c]);
+      gy[c] = r1_h * basis_sum<RowGy<N, q>, NDOF, S::TINY[c]>(co[c]);
+    });
   }
 
   __device__ static void run(const hype_launch& L, int tile_id, double* lds, int lane, int wave) {
@@ -254,7 +296,15 @@ struct Tile {
     const int nx = I->nx, ny = I->ny;
     const int bcL = I->bc[0], bcR = I->bc[1], bcB = I->bc[2], bcT = I->bc[3];
     const double r1_h = I->r1_h;
-    const Eos eos{I->g1, I->g2, I->p1, I->p2, (I->quirks & HYPE_QUIRK_BN_P2_IS_PHI) != 0};
+    Eos eos{I->g1, I->g2, I->p1, I->p2, (I->quirks & HYPE_QUIRK_BN_P2_IS_PHI) != 0, 1.0, 1.0, 1.0, 1.0};
+    if constexpr (PRIM) {
+      double d1, d2;
+      S::energy_den(eos, d1, d2);
+      eos.d1 = uniform(d1);
+      eos.d2 = uniform(d2);
+      eos.y1 = uniform(recip_nr(d1));
+      eos.y2 = uniform(recip_nr(d2));
+    }
     // the first tile of an instance writes its time state (lower wave only)
     const bool leader = (T.flags & 1) != 0 && wave == 0;
     const int mode = L.mode;
@@ -467,7 +517,9 @@ struct Tile {
 
     // ---- carried state -------------------------------------------------
     double topPrev[NGF][NV];
-    double topA[NGF];  // a_sq handed over with topPrev (negative: none)
+    double topA[NGF];  // a_sq handed over with topPrev
+    // the face sums G, E (and Fx, Dx) of most components are kept unscaled (PLAIN
+    // says which are not)
     double Gprev[NV], Eprev[NV], xpartPrev[NV], ncpPrev[NV];
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
@@ -479,39 +531,42 @@ struct Tile {
       for (int q = 0; q < NGF; ++q) topPrev[q][c] = 0.0;
     }
 #pragma unroll
-    for (int q = 0; q < NGF; ++q) topA[q] = -1.0;
-    double smax = 0.0;
+    for (int q = 0; q < NGF; ++q) topA[q] = 0.0;
+    double smax_x = 0.0, smax_y = 0.0;  // largest wave speeds, over all lanes (masked at the end)
     unsigned long long err = ~0ull;
     const int seq = (mode == HYPE_MODE_STAGE) ? L.stage + 1 : 0;
-    const double WF = Qd::WF, WV = Qd::WV;
 
-    // flux + jump at the y-face below row fr from the values either side
+    // an inadmissible state at face point q of a face (key of the face's point
+    // 0); the states are examined again, which nothing but this rare path pays
+    // for
+    auto report = [&](long key0, int q, const double* Lv, const double* Rv, bool mine, bool bad) {
+      if (mine && bad) {
+        const Bad b = riemann_diag<S, PRIM>(eos, Lv, Rv);
+        const unsigned long long pk = pack_err(seq, key0 + q, b.kind, b.val, I->keybits);
+        if (b.kind && pk < err) err = pk;
+      }
+    };
+    // flux + jump sums at the y-face below row fr from the values either side
     // (lower side: top values of row fr-1; upper side: bottom values of fr)
     auto yface = [&](const double (&Lv)[NGF][NV], const double (&Rv)[NGF][NV], const double* aL, const double* aR,
                      int fr, double* G, double* E) {
-#pragma unroll
-      for (int c = 0; c < NV; ++c) {
-        G[c] = 0.0;
-        E[c] = 0.0;
-      }
+      bool bad[NGF], any = false;
 #pragma unroll
       for (int q = 0; q < NGF; ++q) {
-        double Fq[NV], Dq[NV];
-        Bad b{0, 0.0};
-        const double sp = riemann<S, PRIM, 1>(eos, Lv[q], Rv[q], Fq, Dq, b, aL[q], aR[q]);
-        if (owned) {
-          if (sp > smax) smax = sp;
-          if (b.kind) {
-            const long key = (long)ny * (nx + 1) * NGF + ((long)fr * nx + col) * NGF + q;
-            const unsigned long long pk = pack_err(seq, key, b.kind, b.val, I->keybits);
-            if (pk < err) err = pk;
-          }
+        double A[NV], D[NV];
+        const double sp = riemann<S, PRIM, ACACHE, 1>(eos, Lv[q], Rv[q], A, D, bad[q], aL[q], aR[q]);
+        smax_y = fmax(smax_y, sp);
+        any |= bad[q];
+        if constexpr (CHECK_EACH) {
+          if (__builtin_expect(__ballot(bad[q]) != 0, 0))
+            report((long)ny * (nx + 1) * NGF + ((long)fr * nx + col) * NGF, q, Lv[q], Rv[q], owned, bad[q]);
         }
+        add_point<1>(q, A, D, G, E);
+      }
+      if (!CHECK_EACH && __builtin_expect(__ballot(any) != 0, 0)) {
 #pragma unroll
-        for (int c = 0; c < NV; ++c) {
-          G[c] = G[c] + WF * Fq[c];
-          if (S::DNZ[c]) E[c] = E[c] + WF * Dq[c];
-        }
+        for (int q = 0; q < NGF; ++q)
+          report((long)ny * (nx + 1) * NGF + ((long)fr * nx + col) * NGF, q, Lv[q], Rv[q], owned, bad[q]);
       }
     };
 
@@ -553,12 +608,10 @@ struct Tile {
                       const double* xp, const double* nc, bool wr) {
       const size_t idx = ((size_t)row * nx + col) * NV;
       double rhs[NV];
-#pragma unroll
-      for (int c = 0; c < NV; ++c) {
-        const double Y = Gt[c] - Gb[c] + 0.5 * (Et[c] + Eb[c]);
-        const double t = xp[c] - r1_h * Y;
+      static_for<NV>([&](auto c) {
+        const double t = xp[c] - face_diff<1, c>(r1_h, Gt[c], Gb[c], Et[c], Eb[c]);
         rhs[c] = ((S::HAS_NCP && S::DNZ[c]) ? nc[c] : 0.0) + t;
-      }
+      });
       if (mode == HYPE_MODE_RHS) {
 #pragma unroll
         for (int c = 0; c < NV; ++c) put_out(rhs[c], Out, idx + c, 0, c);
@@ -645,8 +698,7 @@ struct Tile {
 
       // ---- reconstruction: modal coefficients of every component --------
       double co[NV][NDOF];
-#pragma unroll
-      for (int c = 0; c < NV; ++c) {
+      static_for<NV>([&](auto c) {
         double ux[5], uy[5], ud[5];
         ux[0] = W_(s0, c, cw - 2);
         ux[1] = W_(s0, c, cw - 1);
@@ -663,8 +715,8 @@ struct Tile {
         ud[2] = W_(sm1, c, cw + 1);
         ud[3] = W_(sp1, c, cw - 1);
         ud[4] = W_(sm1, c, cw - 1);
-        reconstruct<N>(ux, uy, ud, co[c]);
-      }
+        reconstruct<N, S::TINY[c]>(ux, uy, ud, co[c]);
+      });
       // values at the nodes, which are also the face quadrature points
       // (rhs_function_prim.c:382-388, 425-440; the same points, hype.c:207-229)
       double fv[NNODE][NV];
@@ -695,7 +747,7 @@ struct Tile {
         at_nodes(co, fv);
         if constexpr (ACACHE) {
 #pragma unroll
-          for (int p = 0; p < NNODE; ++p) an[p] = -1.0;  // new values: the flux computes a_sq itself
+          for (int p = 0; p < NNODE; ++p) an[p] = S::sound_sq_prim(eos, fv[p]);
         }
       }
       if (L.fallback && ownedRow && owned) gmem(L.fallback)[(size_t)r * nx + col] = (unsigned char)(!pad);
@@ -729,8 +781,17 @@ struct Tile {
             S::template vol_ncp<PRIM>(eos, V, gx, gy, B);
 #pragma unroll
             for (int c = 0; c < NV; ++c)
-              if (S::DNZ[c]) ncp[c] = ncp[c] + -WV * B[c];
+              if (S::DNZ[c]) {
+                if (S::JUMP_TINY[c])
+                  ncp[c] = ncp[c] + -Qd::WV * B[c];
+                else
+                  ncp[c] = q == 0 ? B[c] : ncp[c] + B[c];
+              }
           });
+          // the weight, a power of two, once for the sum; +0 for a zero sum
+#pragma unroll
+          for (int c = 0; c < NV; ++c)
+            if (S::DNZ[c] && !S::JUMP_TINY[c]) ncp[c] = fma(-Qd::WV, ncp[c], 0.0);
         }
       }
 
@@ -739,48 +800,44 @@ struct Tile {
       double xpart[NV];
       {
         double Fx[NV], Dx[NV];
+        bool bad[NGF], any = false;
 #pragma unroll
         for (int c = 0; c < NV; ++c) {
           Fx[c] = 0.0;
           Dx[c] = 0.0;
         }
+        double vl[NGF][NV];
 #pragma unroll
         for (int q = 0; q < NGF; ++q) {
-          double vl[NV], vr[NV], Fq[NV], Dq[NV];
 #pragma unroll
-          for (int c = 0; c < NV; ++c) {
-            vl[c] = lane_from_left(fv[Qd::R(q)][c]);
-            vr[c] = fv[Qd::L(q)][c];
-          }
-          double al = -1.0, ar = -1.0;
+          for (int c = 0; c < NV; ++c) vl[q][c] = lane_from_left(fv[Qd::R(q)][c]);
+          bad[q] = false;
+          double al = 0.0, ar = 0.0;
           if constexpr (ACACHE) {
             al = lane_from_left(an[Qd::R(q)]);
             ar = an[Qd::L(q)];
           }
           if (ownedRow) {
-            Bad b{0, 0.0};
-            const double s = riemann<S, PRIM, 0>(eos, vl, vr, Fq, Dq, b, al, ar);
-            if (xlane) {
-              if (s > smax) smax = s;
-              if (b.kind) {
-                const long key = ((long)r * (nx + 1) + col) * NGF + q;
-                const unsigned long long pk = pack_err(seq, key, b.kind, b.val, I->keybits);
-                if (pk < err) err = pk;
-              }
+            double A[NV], D[NV];
+            const double s = riemann<S, PRIM, ACACHE, 0>(eos, vl[q], fv[Qd::L(q)], A, D, bad[q], al, ar);
+            smax_x = fmax(smax_x, s);
+            any |= bad[q];
+            if constexpr (CHECK_EACH) {
+              if (__builtin_expect(__ballot(bad[q]) != 0, 0))
+                report(((long)r * (nx + 1) + col) * NGF, q, vl[q], fv[Qd::L(q)], xlane, bad[q]);
             }
-#pragma unroll
-            for (int c = 0; c < NV; ++c) {
-              Fx[c] = Fx[c] + WF * Fq[c];
-              if (S::DNZ[c]) Dx[c] = Dx[c] + WF * Dq[c];
-            }
+            add_point<0>(q, A, D, Fx, Dx);
           }
         }
+        if (!CHECK_EACH && __builtin_expect(__ballot(any) != 0, 0)) {
 #pragma unroll
-        for (int c = 0; c < NV; ++c) {
-          const double Fr = lane_from_right(Fx[c]);
-          const double Dr = S::DNZ[c] ? lane_from_right(Dx[c]) : 0.0;
-          xpart[c] = -r1_h * (Fr - Fx[c] + 0.5 * (Dr + Dx[c]));
+          for (int q = 0; q < NGF; ++q)
+            report(((long)r * (nx + 1) + col) * NGF, q, vl[q], fv[Qd::L(q)], xlane, bad[q]);
         }
+        static_for<NV>([&](auto c) {
+          const double Dr = S::DNZ[c] ? lane_from_right(Dx[c]) : 0.0;
+          xpart[c] = -face_diff<0, c>(r1_h, lane_from_right(Fx[c]), Fx[c], Dr, Dx[c]);
+        });
       }
 
       // ---- y-face r-1/2 (rhs_function_prim.c:537-585) --------------------
@@ -788,7 +845,7 @@ struct Tile {
       if (doY) {
         double an_b[NGF];
 #pragma unroll
-        for (int q = 0; q < NGF; ++q) an_b[q] = ACACHE ? an[Qd::B(q)] : -1.0;
+        for (int q = 0; q < NGF; ++q) an_b[q] = ACACHE ? an[Qd::B(q)] : 0.0;
         double fvb[NGF][NV];
 #pragma unroll
         for (int q = 0; q < NGF; ++q)
@@ -808,7 +865,7 @@ struct Tile {
           for (int q = 0; q < NGF; ++q) {
 #pragma unroll
             for (int c = 0; c < NV; ++c) X_(1, q, c) = fv[Qd::B(q)][c];
-            X_(1, q, NV) = ACACHE ? an[Qd::B(q)] : -1.0;
+            X_(1, q, NV) = ACACHE ? an[Qd::B(q)] : 0.0;
           }
         }
         if (upper && r == ym + 1) {  // so does the assembly of row ym
@@ -844,6 +901,9 @@ struct Tile {
     }
 
     const bool want_smax = (mode != HYPE_MODE_STAGE) || last_stage;
+    // the faces that count: x-faces of the owned columns, y-faces of owned cells
+    auto lane_smax = [&]() { return fmax(xlane ? smax_x : 0.0, owned ? smax_y : 0.0); };
+    double other_smax = 0.0;
 
     // ---- the two halves of a split tile meet at face ym-1/2 -----------------
     if constexpr (PAIR) {
@@ -861,14 +921,13 @@ struct Tile {
         // both waves solve the same middle face, and the upper wave adds no
         // other face, so the lower wave's maximum then covers the tile
         if constexpr (COMBINE) {
-          const double um = (want_smax && upper) ? wave_max(smax) : 0.0;
+          const double um = (want_smax && upper) ? wave_max(lane_smax()) : 0.0;
           if (want_smax && upper && lane == 0) *pair_smax = um;
         }
         __syncthreads();
         if constexpr (COMBINE) {
           if (want_smax && !upper) {
-            const double pm = *pair_smax;
-            if (pm > smax) smax = pm;
+            other_smax = *pair_smax;
           }
         }
         double lo[NGF][NV], hi[NGF][NV], alo[NGF], ahi[NGF];
@@ -902,7 +961,7 @@ struct Tile {
 
     // ---- CFL maximum and error word ----------------------------------------
     if (want_smax && !(COMBINE && split && upper)) {
-      const double m = wave_max(smax);
+      const double m = wave_max(fmax(lane_smax(), other_smax));
       if (lane == 0) {
         unsigned long long* slotp =
             (mode == HYPE_MODE_RHS) ? &st->smax_rhs : (mode == HYPE_MODE_PRIME ? &st->smax[st->step & 1] : &st->smax[(cur + 1) & 1]);
