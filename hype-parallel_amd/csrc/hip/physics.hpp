@@ -98,14 +98,14 @@ struct Euler {
   static constexpr bool FZERO[NV] = {false, false, false, false};
   static constexpr bool TINY[NV] = {false, true, true, false};
   static constexpr bool JUMP_TINY[NV] = {false, false, false, false};
-  __device__ static void energy_den(const Eos& e, double& d1, double& d2) {
+  __device__ static __forceinline__ void energy_den(const Eos& e, double& d1, double& d2) {
     d1 = e.g1 - 1.0;
     d2 = 1.0;
   }
 
   // euler.c:14-23
-  __device__ static void cons2prim(const Eos& e, const double* Q, double* V) {
-    double irho = 1.0 / Q[0];
+  __device__ static __forceinline__ void cons2prim(const Eos& e, const double* Q, double* V) {
+    double irho = fdiv(1.0, Q[0]);
     V[0] = Q[0];
     V[1] = irho * Q[1];
     V[2] = irho * Q[2];
@@ -113,9 +113,9 @@ struct Euler {
   }
   // flux and wave speed of a conserved state (euler.c:44-84)
   template <int DIR>
-  __device__ static double side_cons(const Eos& e, const double* Q, double* F, bool& bad) {
+  __device__ static __forceinline__ double side_cons(const Eos& e, const double* Q, double* F, bool& bad) {
     double rho = Q[0];
-    double irho = 1.0 / rho;
+    double irho = fdiv(1.0, rho);
     double u = irho * Q[1];
     double v = irho * Q[2];
     double un = normal<DIR>(u, v);
@@ -130,9 +130,9 @@ struct Euler {
     return fabs(un) + sqrt_adm(e.g1 * p * irho);
   }
   // which check of the flux a state fails first (euler.c:60-70)
-  __device__ static void diag_cons(const Eos& e, const double* Q, Bad& b) {
+  __device__ static __forceinline__ void diag_cons(const Eos& e, const double* Q, Bad& b) {
     double rho = Q[0];
-    double irho = 1.0 / rho;
+    double irho = fdiv(1.0, rho);
     double u = irho * Q[1];
     double v = irho * Q[2];
     double p = (e.g1 - 1.0) * fma(-0.5, rho * (u * u + v * v), Q[3]);
@@ -142,7 +142,7 @@ struct Euler {
   // flux, wave speed and conserved variables of a primitive state
   // (euler.c:29-38, 197-236)
   template <int DIR>
-  __device__ static double side_prim(const Eos& e, const double* V, double* F, double* Q, bool& bad) {
+  __device__ static __forceinline__ double side_prim(const Eos& e, const double* V, double* F, double* Q, bool& bad) {
     double rho = V[0];
     double u = V[1];
     double v = V[2];
@@ -159,18 +159,18 @@ struct Euler {
     Q[1] = rho * u;
     Q[2] = rho * v;
     Q[3] = E;
-    return fabs(un) + sqrt_adm(e.g1 * p / rho);
+    return fabs(un) + sqrt_adm(fdiv(e.g1 * p, rho));
   }
   // euler.c:212-222
-  __device__ static void diag_prim(const Eos&, const double* V, Bad& b) {
+  __device__ static __forceinline__ void diag_prim(const Eos&, const double* V, Bad& b) {
     if (V[0] < RHO_FLOOR) b.set(1, V[0]);
     if (V[3] < PRS_FLOOR) b.set(2, V[3]);
   }
   // euler.c:169-191
-  __device__ static bool pad(const Eos& e, const double* Q) {
+  __device__ static __forceinline__ bool pad(const Eos& e, const double* Q) {
     bool ok = true;
     double rho = Q[0];
-    double irho = 1.0 / rho;
+    double irho = fdiv(1.0, rho);
     double u = irho * Q[1];
     double v = irho * Q[2];
     double p = (e.g1 - 1.0) * fma(-0.5, rho * (u * u + v * v), Q[3]);
@@ -179,19 +179,19 @@ struct Euler {
     return ok;
   }
   // euler.c:292-310
-  __device__ static bool pad_prim(const Eos&, const double* V) {
+  __device__ static __forceinline__ bool pad_prim(const Eos&, const double* V) {
     bool ok = true;
     if (V[0] < RHO_FLOOR) ok = false;
     if (V[3] < PRS_FLOOR) ok = false;
     return ok;
   }
   template <bool PRIM>
-  __device__ static void vol_ncp(const Eos&, const double*, const double*, const double*, double* B) {
+  __device__ static __forceinline__ void vol_ncp(const Eos&, const double*, const double*, const double*, double* B) {
     for (int c = 0; c < NV; ++c) B[c] = 0.0;
   }
   // face jump term: identically zero (euler.c:142-148, 278-286)
   template <bool PRIM, int DIR>
-  __device__ static void ncp_face(const Eos&, const double*, const double*, double* D) {
+  __device__ static __forceinline__ void ncp_face(const Eos&, const double*, const double*, double* D) {
     for (int c = 0; c < NV; ++c) D[c] = 0.0;
   }
 };
@@ -221,37 +221,39 @@ struct Kapila {
   static constexpr bool FZERO[NV] = {false, false, false, false, false, true};
   static constexpr bool TINY[NV] = {false, false, true, true, false, false};
   static constexpr bool JUMP_TINY[NV] = {false, false, false, false, false, true};
-  __device__ static void energy_den(const Eos& e, double& d1, double& d2) {
+  __device__ static __forceinline__ void energy_den(const Eos& e, double& d1, double& d2) {
     d1 = (e.g1 - 1.0) * (e.g2 - 1.0);
     d2 = 1.0;
   }
 
   // pressure of a conserved state (kapila_5eqn.c:22-30)
-  __device__ static double pressure(const Eos& e, const double* Q, double rho, double u, double v, double alpha_2) {
+  __device__ static __forceinline__ double pressure(const Eos& e, const double* Q, double rho, double u, double v,
+                                                    double alpha_2) {
     double alpha_1 = Q[5];
     double en = fma(-0.5, rho * (u * u + v * v), Q[4]);
     double G1m1 = e.g1 - 1.0;
     double G2m1 = e.g2 - 1.0;
-    return (en * G1m1 * G2m1 - alpha_1 * e.g1 * e.p1 * G2m1 - alpha_2 * e.g2 * e.p2 * G1m1) /
-           (alpha_1 * G2m1 + alpha_2 * G1m1);
+    return fdiv(en * G1m1 * G2m1 - alpha_1 * e.g1 * e.p1 * G2m1 - alpha_2 * e.g2 * e.p2 * G1m1,
+                alpha_1 * G2m1 + alpha_2 * G1m1);
   }
   // the mixture's squared speed of sound (kapila_5eqn.c:89-94, 347-352)
-  __device__ static double sound_sq(const Eos& e, double rho_1, double rho_2, double rho, double p, double alpha_1,
+  __device__ static __forceinline__ double sound_sq(const Eos& e, double rho_1, double rho_2, double rho, double p,
+                                                    double alpha_1,
                                     double alpha_2) {
-    double a1_sq = e.g1 * (p + e.p1) / rho_1;
-    double a2_sq = e.g2 * (p + e.p2) / rho_2;
-    return (rho_1 * a1_sq * rho_2 * a2_sq) / (rho * (alpha_2 * rho_1 * a1_sq + alpha_1 * rho_2 * a2_sq));
+    double a1_sq = fdiv(e.g1 * (p + e.p1), rho_1);
+    double a2_sq = fdiv(e.g2 * (p + e.p2), rho_2);
+    return fdiv(rho_1 * a1_sq * rho_2 * a2_sq, rho * (alpha_2 * rho_1 * a1_sq + alpha_1 * rho_2 * a2_sq));
   }
 
   // kapila_5eqn.c:14-35
-  __device__ static void cons2prim(const Eos& e, const double* Q, double* V) {
+  __device__ static __forceinline__ void cons2prim(const Eos& e, const double* Q, double* V) {
     double alpha_1 = Q[5];
     double alpha_2 = 1.0 - alpha_1;
     double rho = Q[0] + Q[1];
-    double u = Q[2] / rho;
-    double v = Q[3] / rho;
-    V[0] = Q[0] / alpha_1;
-    V[1] = Q[1] / alpha_2;
+    double u = fdiv(Q[2], rho);
+    double v = fdiv(Q[3], rho);
+    V[0] = fdiv(Q[0], alpha_1);
+    V[1] = fdiv(Q[1], alpha_2);
     V[2] = u;
     V[3] = v;
     V[4] = pressure(e, Q, rho, u, v, alpha_2);
@@ -259,14 +261,14 @@ struct Kapila {
   }
   // flux and wave speed of a conserved state (kapila_5eqn.c:67-113)
   template <int DIR>
-  __device__ static double side_cons(const Eos& e, const double* Q, double* F, bool& bad) {
+  __device__ static __forceinline__ double side_cons(const Eos& e, const double* Q, double* F, bool& bad) {
     double alpha_1 = Q[5];
     double alpha_2 = 1.0 - alpha_1;
-    double rho_1 = Q[0] / alpha_1;
-    double rho_2 = Q[1] / alpha_2;
+    double rho_1 = fdiv(Q[0], alpha_1);
+    double rho_2 = fdiv(Q[1], alpha_2);
     double rho = Q[0] + Q[1];
-    double u = Q[2] / rho;
-    double v = Q[3] / rho;
+    double u = fdiv(Q[2], rho);
+    double v = fdiv(Q[3], rho);
     double E = Q[4];
     double p = pressure(e, Q, rho, u, v, alpha_2);
     double un = normal<DIR>(u, v);
@@ -280,22 +282,23 @@ struct Kapila {
     F[5] = 0.0;
     return fabs(un) + sqrt_adm(a_sq);
   }
-  __device__ static double sound_sq_cons(const Eos& e, const double* Q) {
+  __device__ static __forceinline__ double sound_sq_cons(const Eos& e, const double* Q) {
     double alpha_1 = Q[5];
     double alpha_2 = 1.0 - alpha_1;
     double rho = Q[0] + Q[1];
-    double u = Q[2] / rho;
-    double v = Q[3] / rho;
-    return sound_sq(e, Q[0] / alpha_1, Q[1] / alpha_2, rho, pressure(e, Q, rho, u, v, alpha_2), alpha_1, alpha_2);
+    double u = fdiv(Q[2], rho);
+    double v = fdiv(Q[3], rho);
+    return sound_sq(e, fdiv(Q[0], alpha_1), fdiv(Q[1], alpha_2), rho, pressure(e, Q, rho, u, v, alpha_2), alpha_1,
+                    alpha_2);
   }
   // kapila_5eqn.c:95-99
-  __device__ static void diag_cons(const Eos& e, const double* Q, Bad& b) {
+  __device__ static __forceinline__ void diag_cons(const Eos& e, const double* Q, Bad& b) {
     const double a_sq = sound_sq_cons(e, Q);
     if (a_sq < PRS_FLOOR) b.set(3, a_sq);
   }
   // a_sq of a primitive state; the admissibility check (kapila_5eqn.c:468-470)
   // and the flux (:347-352) compute the same expression
-  __device__ static double sound_sq_prim(const Eos& e, const double* V) {
+  __device__ static __forceinline__ double sound_sq_prim(const Eos& e, const double* V) {
     double alpha_1 = V[5];
     double alpha_2 = 1.0 - alpha_1;
     double rho = alpha_1 * V[0] + alpha_2 * V[1];
@@ -304,7 +307,8 @@ struct Kapila {
   // flux, wave speed and conserved variables of a primitive state whose a_sq
   // is given (kapila_5eqn.c:41-61, 326-371)
   template <int DIR>
-  __device__ static double side_prim_a(const Eos& e, const double* V, double a_sq, double* F, double* Q, bool& bad) {
+  __device__ static __forceinline__ double side_prim_a(const Eos& e, const double* V, double a_sq, double* F,
+                                                       double* Q, bool& bad) {
     double alpha_1 = V[5];
     double alpha_2 = 1.0 - alpha_1;
     double m1 = alpha_1 * V[0];
@@ -338,16 +342,16 @@ struct Kapila {
     return fabs(un) + sqrt_adm(a_sq);
   }
   template <int DIR>
-  __device__ static double side_prim(const Eos& e, const double* V, double* F, double* Q, bool& bad) {
+  __device__ static __forceinline__ double side_prim(const Eos& e, const double* V, double* F, double* Q, bool& bad) {
     return side_prim_a<DIR>(e, V, sound_sq_prim(e, V), F, Q, bad);
   }
   // kapila_5eqn.c:353-357
-  __device__ static void diag_prim(const Eos& e, const double* V, Bad& b) {
+  __device__ static __forceinline__ void diag_prim(const Eos& e, const double* V, Bad& b) {
     const double a_sq = sound_sq_prim(e, V);
     if (a_sq < PRS_FLOOR) b.set(3, a_sq);
   }
   // kapila_5eqn.c:247-283 (alpha_1 test of :278 kept)
-  __device__ static bool pad(const Eos& e, const double* Q) {
+  __device__ static __forceinline__ bool pad(const Eos& e, const double* Q) {
     const double a_sq = sound_sq_cons(e, Q);
     if (Q[0] + Q[1] < RHO_FLOOR) return false;
     if (a_sq < PRS_FLOOR) return false;
@@ -355,7 +359,7 @@ struct Kapila {
     return true;
   }
   // kapila_5eqn.c:450-479; also returns the a_sq it computes (for side_prim_a)
-  __device__ static bool pad_prim_a(const Eos& e, const double* V, double& a_out) {
+  __device__ static __forceinline__ bool pad_prim_a(const Eos& e, const double* V, double& a_out) {
     double alpha_1 = V[5];
     double alpha_2 = 1.0 - alpha_1;
     double rho = alpha_1 * V[0] + alpha_2 * V[1];
@@ -366,13 +370,13 @@ struct Kapila {
     if (alpha_1 < 0.0 || alpha_1 > 1.0) return false;
     return true;
   }
-  __device__ static bool pad_prim(const Eos& e, const double* V) {
+  __device__ static __forceinline__ bool pad_prim(const Eos& e, const double* V) {
     double a_sq;
     return pad_prim_a(e, V, a_sq);
   }
   // B*grad for the primitive path, comp 5 only (kapila_5eqn.c:417-444);
   // arguments: V (6 values), alpha_x, alpha_y, u_x, v_y
-  __device__ static double ncp5_prim(const Eos& e, const double* V, double phi_x, double phi_y,
+  __device__ static __forceinline__ double ncp5_prim(const Eos& e, const double* V, double phi_x, double phi_y,
                                      double u_x, double v_y) {
     double alpha_1 = V[5];
     double alpha_2 = 1.0 - alpha_1;
@@ -381,27 +385,29 @@ struct Kapila {
     double u = V[2];
     double v = V[3];
     double p = V[4];
-    double a_1_sq = e.g1 * (p + e.p1) / rho_1;
-    double a_2_sq = e.g2 * (p + e.p2) / rho_2;
-    double K = (alpha_1 * alpha_2 * (rho_2 * a_2_sq - rho_1 * a_1_sq)) /
-               (alpha_1 * rho_2 * a_2_sq + alpha_2 * rho_1 * a_1_sq);
+    double a_1_sq = fdiv(e.g1 * (p + e.p1), rho_1);
+    double a_2_sq = fdiv(e.g2 * (p + e.p2), rho_2);
+    double K = fdiv(alpha_1 * alpha_2 * (rho_2 * a_2_sq - rho_1 * a_1_sq),
+                    alpha_1 * rho_2 * a_2_sq + alpha_2 * rho_1 * a_1_sq);
     return u * phi_x + v * phi_y - K * (u_x + v_y);
   }
   // B*grad for the conservative path, comp 5 only (kapila_5eqn.c:164-198);
   // gx, gy: gradients of all components
-  __device__ static double ncp5_cons(const Eos& e, const double* Q, const double* gx, const double* gy) {
+  __device__ static __forceinline__ double ncp5_cons(const Eos& e, const double* Q, const double* gx,
+                                                     const double* gy) {
     double alpha_1 = Q[5];
     double alpha_2 = 1.0 - alpha_1;
-    double rho_1 = Q[0] / alpha_1;
-    double rho_2 = Q[1] / alpha_2;
+    double rho_1 = fdiv(Q[0], alpha_1);
+    double rho_2 = fdiv(Q[1], alpha_2);
     double rho = Q[0] + Q[1];
-    double irho = 1.0 / rho;
-    double u = Q[2] / rho;
-    double v = Q[3] / rho;
+    double irho = fdiv(1.0, rho);
+    double u = fdiv(Q[2], rho);
+    double v = fdiv(Q[3], rho);
     double p = pressure(e, Q, rho, u, v, alpha_2);
-    double a1_sq = e.g1 * (p + e.p1) / rho_1;
-    double a2_sq = e.g2 * (p + e.p2) / rho_2;
-    double K = alpha_1 * alpha_2 * (rho_2 * a2_sq - rho_1 * a1_sq) / (alpha_1 * rho_2 * a2_sq + alpha_2 * rho_1 * a1_sq);
+    double a1_sq = fdiv(e.g1 * (p + e.p1), rho_1);
+    double a2_sq = fdiv(e.g2 * (p + e.p2), rho_2);
+    double K = fdiv(alpha_1 * alpha_2 * (rho_2 * a2_sq - rho_1 * a1_sq),
+                    alpha_1 * rho_2 * a2_sq + alpha_2 * rho_1 * a1_sq);
     double alpha1_x = gx[5];
     double alpha1_y = gy[5];
     double u_x = irho * irho * (gx[2] * rho - Q[2] * (gx[0] + gx[1]));
@@ -410,7 +416,8 @@ struct Kapila {
   }
   // volume term B(V) grad V at a quadrature point (rhs_function_prim.c:474)
   template <bool PRIM>
-  __device__ static void vol_ncp(const Eos& e, const double* V, const double* gx, const double* gy, double* B) {
+  __device__ static __forceinline__ void vol_ncp(const Eos& e, const double* V, const double* gx, const double* gy,
+                                                 double* B) {
     for (int c = 0; c < 5; ++c) B[c] = 0.0;
     if (PRIM)
       B[5] = ncp5_prim(e, V, gx[5], gy[5], gx[2], gy[3]);
@@ -424,7 +431,7 @@ struct Kapila {
   // mean's factors 1/2 are kept out of the densities, where they cancel exactly
   // (rho_k a_k^2 = (2 rho_k)(a_k^2 / 2))
   template <bool PRIM, int DIR>
-  __device__ static void ncp_face(const Eos& e, const double* L, const double* R, double* D) {
+  __device__ static __forceinline__ void ncp_face(const Eos& e, const double* L, const double* R, double* D) {
     for (int c = 0; c < 5; ++c) D[c] = 0.0;
     if (PRIM) {
       constexpr int n = 2 + DIR;
@@ -435,9 +442,9 @@ struct Kapila {
       double as = R[5] + L[5];
       double alpha_1 = 0.5 * as;
       double alpha_2 = fma(-0.5, as, 1.0);
-      double a_1_sq = e.g1 * fma(0.5, ps, e.p1) / r1;  // half of them
-      double a_2_sq = e.g2 * fma(0.5, ps, e.p2) / r2;
-      double K = (alpha_1 * alpha_2 * (r2 * a_2_sq - r1 * a_1_sq)) / (alpha_1 * r2 * a_2_sq + alpha_2 * r1 * a_1_sq);
+      double a_1_sq = fdiv(e.g1 * fma(0.5, ps, e.p1), r1);  // half of them
+      double a_2_sq = fdiv(e.g2 * fma(0.5, ps, e.p2), r2);
+      double K = fdiv(alpha_1 * alpha_2 * (r2 * a_2_sq - r1 * a_1_sq), alpha_1 * r2 * a_2_sq + alpha_2 * r1 * a_1_sq);
       D[5] = un * (R[5] - L[5]) - K * (R[n] - L[n]);
     } else {
       constexpr double nx = DIR == 0 ? 1.0 : 0.0, ny = DIR == 0 ? 0.0 : 1.0;
@@ -471,52 +478,53 @@ struct BN {
   static constexpr bool FZERO[NV] = {false, false, false, false, false, false, false, false, true};
   static constexpr bool TINY[NV] = {false, true, true, false, false, true, true, false, false};
   static constexpr bool JUMP_TINY[NV] = {false, false, false, false, false, false, false, false, false};
-  __device__ static void energy_den(const Eos& e, double& d1, double& d2) {
+  __device__ static __forceinline__ void energy_den(const Eos& e, double& d1, double& d2) {
     d1 = e.g1 - 1.0;
     d2 = e.g2 - 1.0;
   }
 
   // pressure of a phase from its density, velocity and total energy per volume
   // (baer_nunziato.c:29-30)
-  __device__ static double pressure(double g, double pi, double rho, double u, double v, double E) {
+  __device__ static __forceinline__ double pressure(double g, double pi, double rho, double u, double v, double E) {
     return (g - 1.0) * fma(-0.5, rho * (u * u + v * v), E) - g * pi;
   }
   // baer_nunziato.c:14-41
-  __device__ static void cons2prim(const Eos& e, const double* Q, double* V) {
+  __device__ static __forceinline__ void cons2prim(const Eos& e, const double* Q, double* V) {
     double phi_1 = Q[8];
     double phi_2 = 1.0 - Q[8];
-    double rho_1 = Q[0] / phi_1;
-    double rho_2 = Q[4] / phi_2;
-    double u_1 = Q[1] / Q[0];
-    double v_1 = Q[2] / Q[0];
-    double u_2 = Q[5] / Q[4];
-    double v_2 = Q[6] / Q[4];
+    double rho_1 = fdiv(Q[0], phi_1);
+    double rho_2 = fdiv(Q[4], phi_2);
+    double u_1 = fdiv(Q[1], Q[0]);
+    double v_1 = fdiv(Q[2], Q[0]);
+    double u_2 = fdiv(Q[5], Q[4]);
+    double v_2 = fdiv(Q[6], Q[4]);
     V[0] = rho_1;
     V[1] = u_1;
     V[2] = v_1;
-    V[3] = pressure(e.g1, e.p1, rho_1, u_1, v_1, Q[3] / phi_1);
+    V[3] = pressure(e.g1, e.p1, rho_1, u_1, v_1, fdiv(Q[3], phi_1));
     V[4] = rho_2;
     V[5] = u_2;
     V[6] = v_2;
-    V[7] = pressure(e.g2, e.p2, rho_2, u_2, v_2, Q[7] / phi_2);
+    V[7] = pressure(e.g2, e.p2, rho_2, u_2, v_2, fdiv(Q[7], phi_2));
     V[8] = phi_1;
   }
   // baer_nunziato.c:47-60
-  __device__ static void prim2cons(const Eos& e, const double* V, double* Q) {
+  __device__ static __forceinline__ void prim2cons(const Eos& e, const double* V, double* Q) {
     Q[0] = V[8] * V[0];
     Q[1] = Q[0] * V[1];
     Q[2] = Q[0] * V[2];
-    Q[3] = Q[0] * fma(0.5, V[1] * V[1] + V[2] * V[2], (V[3] + e.g1 * e.p1) / (V[0] * (e.g1 - 1.0)));
+    Q[3] = Q[0] * fma(0.5, V[1] * V[1] + V[2] * V[2], fdiv(V[3] + e.g1 * e.p1, V[0] * (e.g1 - 1.0)));
     Q[4] = (1.0 - V[8]) * V[4];
     Q[5] = Q[4] * V[5];
     Q[6] = Q[4] * V[6];
-    Q[7] = Q[4] * fma(0.5, V[5] * V[5] + V[6] * V[6], (V[7] + e.g2 * e.p2) / (V[4] * (e.g2 - 1.0)));
+    Q[7] = Q[4] * fma(0.5, V[5] * V[5] + V[6] * V[6], fdiv(V[7] + e.g2 * e.p2, V[4] * (e.g2 - 1.0)));
     Q[8] = V[8];
   }
   // the fluxes and wave speed of the two phases from their primitive variables
   // and total energies (baer_nunziato.c:115-130, 305-320)
   template <int DIR>
-  __device__ static double fluxes(const Eos& e, double phi_1, double rho_1, double u_1, double v_1, double p_1,
+  __device__ static __forceinline__ double fluxes(const Eos& e, double phi_1, double rho_1, double u_1, double v_1,
+                                                  double p_1,
                                   double E_1, double rho_2, double u_2, double v_2, double p_2, double E_2, double* F,
                                   bool& bad) {
     double phi_2 = 1.0 - phi_1;
@@ -534,12 +542,13 @@ struct BN {
     F[6] = phi_2 * add_pressure<DIR, 1>(rho_2 * v_2 * un_2, p_2);
     F[7] = phi_2 * un_2 * (E_2 + p_2);
     F[8] = 0.0;
-    double s_1 = fabs(un_1) + sqrt_adm(e.g1 * ps_1 / rho_1);
-    double s_2 = fabs(un_2) + sqrt_adm(e.g2 * ps_2 / rho_2);
+    double s_1 = fabs(un_1) + sqrt_adm(fdiv(e.g1 * ps_1, rho_1));
+    double s_2 = fabs(un_2) + sqrt_adm(fdiv(e.g2 * ps_2, rho_2));
     return pmax(s_1, s_2);
   }
   // which check a state fails first (baer_nunziato.c:91-113, 281-303)
-  __device__ static void diag(const Eos& e, double rho_1, double p_1, double rho_2, double p_2, Bad& b) {
+  __device__ static __forceinline__ void diag(const Eos& e, double rho_1, double p_1, double rho_2, double p_2,
+                                              Bad& b) {
     if (rho_1 < RHO_FLOOR) b.set(4, rho_1);
     if (rho_2 < RHO_FLOOR) b.set(5, rho_2);
     if ((p_1 + e.p1) < PRS_FLOOR) b.set(6, p_1 + e.p1);
@@ -547,29 +556,29 @@ struct BN {
   }
   // baer_nunziato.c:66-131
   template <int DIR>
-  __device__ static double side_cons(const Eos& e, const double* Q, double* F, bool& bad) {
+  __device__ static __forceinline__ double side_cons(const Eos& e, const double* Q, double* F, bool& bad) {
     double phi_1 = Q[8];
     double phi_2 = 1.0 - Q[8];
-    double rho_1 = Q[0] / phi_1;
-    double rho_2 = Q[4] / phi_2;
-    double u_1 = Q[1] / Q[0];
-    double v_1 = Q[2] / Q[0];
-    double u_2 = Q[5] / Q[4];
-    double v_2 = Q[6] / Q[4];
-    double E_1 = Q[3] / phi_1;
-    double E_2 = Q[7] / phi_2;
+    double rho_1 = fdiv(Q[0], phi_1);
+    double rho_2 = fdiv(Q[4], phi_2);
+    double u_1 = fdiv(Q[1], Q[0]);
+    double v_1 = fdiv(Q[2], Q[0]);
+    double u_2 = fdiv(Q[5], Q[4]);
+    double v_2 = fdiv(Q[6], Q[4]);
+    double E_1 = fdiv(Q[3], phi_1);
+    double E_2 = fdiv(Q[7], phi_2);
     double p_1 = pressure(e.g1, e.p1, rho_1, u_1, v_1, E_1);
     double p_2 = pressure(e.g2, e.p2, rho_2, u_2, v_2, E_2);
     return fluxes<DIR>(e, phi_1, rho_1, u_1, v_1, p_1, E_1, rho_2, u_2, v_2, p_2, E_2, F, bad);
   }
-  __device__ static void diag_cons(const Eos& e, const double* Q, Bad& b) {
+  __device__ static __forceinline__ void diag_cons(const Eos& e, const double* Q, Bad& b) {
     double V[NV];
     cons2prim(e, Q, V);
     diag(e, V[0], V[3], V[4], V[7], b);
   }
   // baer_nunziato.c:256-321
   template <int DIR>
-  __device__ static double side_prim(const Eos& e, const double* V, double* F, double* Q, bool& bad) {
+  __device__ static __forceinline__ double side_prim(const Eos& e, const double* V, double* F, double* Q, bool& bad) {
     double p_1 = V[3];
     double p_2 = e.bn_p2_quirk ? V[8] : V[7];
     double E_1 = fma(0.5, V[0] * (V[1] * V[1] + V[2] * V[2]), div_const(p_1 + e.g1 * e.p1, e.d1, e.y1));
@@ -577,17 +586,17 @@ struct BN {
     prim2cons(e, V, Q);
     return fluxes<DIR>(e, V[8], V[0], V[1], V[2], p_1, E_1, V[4], V[5], V[6], p_2, E_2, F, bad);
   }
-  __device__ static void diag_prim(const Eos& e, const double* V, Bad& b) {
+  __device__ static __forceinline__ void diag_prim(const Eos& e, const double* V, Bad& b) {
     diag(e, V[0], V[3], V[4], e.bn_p2_quirk ? V[8] : V[7], b);
   }
   // baer_nunziato.c:207-250
-  __device__ static bool pad(const Eos& e, const double* Q) {
+  __device__ static __forceinline__ bool pad(const Eos& e, const double* Q) {
     double V[NV];
     cons2prim(e, Q, V);
     return pad_prim(e, V);
   }
   // baer_nunziato.c:350-385
-  __device__ static bool pad_prim(const Eos& e, const double* V) {
+  __device__ static __forceinline__ bool pad_prim(const Eos& e, const double* V) {
     bool ok = true;
     if (V[0] < RHO_FLOOR) ok = false;
     if (V[4] < RHO_FLOOR) ok = false;
@@ -599,7 +608,8 @@ struct BN {
   // B*grad from the interface velocity u_1 and pressure p_2 (DIR: face
   // direction, whose other gradient component is a signed zero; 2: volume term)
   template <int DIR>
-  __device__ static void ncp(double u_I, double v_I, double p_I, double phi_x, double phi_y, double* B) {
+  __device__ static __forceinline__ void ncp(double u_I, double v_I, double p_I, double phi_x, double phi_y,
+                                             double* B) {
     double adv = DIR == 0   ? fma(v_I, phi_y, u_I * phi_x)
                  : DIR == 1 ? fma(u_I, phi_x, v_I * phi_y)
                             : u_I * phi_x + v_I * phi_y;
@@ -615,28 +625,30 @@ struct BN {
   }
   // primitive path (baer_nunziato.c:327-344)
   template <int DIR>
-  __device__ static void ncp_prim(const double* V, double phi_x, double phi_y, double* B) {
+  __device__ static __forceinline__ void ncp_prim(const double* V, double phi_x, double phi_y, double* B) {
     ncp<DIR>(V[1], V[2], V[7], phi_x, phi_y, B);
   }
   // conservative path (baer_nunziato.c:137-165)
   template <int DIR>
-  __device__ static void ncp_cons(const Eos& e, const double* Q, double phi_x, double phi_y, double* B) {
+  __device__ static __forceinline__ void ncp_cons(const Eos& e, const double* Q, double phi_x, double phi_y,
+                                                  double* B) {
     double phi_2 = 1.0 - Q[8];
-    double rho_2 = Q[4] / phi_2;
-    double u_2 = Q[5] / Q[4];
-    double v_2 = Q[6] / Q[4];
-    double p_I = pressure(e.g2, e.p2, rho_2, u_2, v_2, Q[7] / phi_2);
-    ncp<DIR>(Q[1] / Q[0], Q[2] / Q[0], p_I, phi_x, phi_y, B);
+    double rho_2 = fdiv(Q[4], phi_2);
+    double u_2 = fdiv(Q[5], Q[4]);
+    double v_2 = fdiv(Q[6], Q[4]);
+    double p_I = pressure(e.g2, e.p2, rho_2, u_2, v_2, fdiv(Q[7], phi_2));
+    ncp<DIR>(fdiv(Q[1], Q[0]), fdiv(Q[2], Q[0]), p_I, phi_x, phi_y, B);
   }
   template <bool PRIM>
-  __device__ static void vol_ncp(const Eos& e, const double* V, const double* gx, const double* gy, double* B) {
+  __device__ static __forceinline__ void vol_ncp(const Eos& e, const double* V, const double* gx, const double* gy,
+                                                 double* B) {
     if (PRIM)
       ncp_prim<2>(V, gx[8], gy[8], B);
     else
       ncp_cons<2>(e, V, gx[8], gy[8], B);
   }
   template <bool PRIM, int DIR>
-  __device__ static void ncp_face(const Eos& e, const double* L, const double* R, double* D) {
+  __device__ static __forceinline__ void ncp_face(const Eos& e, const double* L, const double* R, double* D) {
     constexpr double nx = DIR == 0 ? 1.0 : 0.0, ny = DIR == 0 ? 0.0 : 1.0;
     double av[NV];
     for (int c = 0; c < NV; ++c) av[c] = 0.5 * (R[c] + L[c]);

@@ -289,7 +289,7 @@ struct Tile {
     });
   }
 
-  __device__ static void run(const hype_launch& L, int tile_id, double* lds, int lane, int wave) {
+  __device__ static __forceinline__ void run(const hype_launch& L, int tile_id, double* lds, int lane, int wave) {
     const hype_tile T = L.tiles[tile_id];
     const hype_inst* I = &L.insts[T.inst];
     hype_dstate* st = I->st;
@@ -999,20 +999,22 @@ __global__ __launch_bounds__(PR ? 2 * HYPE_WAVE : HYPE_WAVE)
   const int lane = (int)threadIdx.x % HYPE_WAVE;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / HYPE_WAVE);
   const int ntiles = L.ntiles_dev ? *L.ntiles_dev : L.ntiles;
-  if (L.grid <= 0) {
-    if ((int)blockIdx.x < ntiles) TT::run(L, blockIdx.x, lds, lane, wave);
-    return;
-  }
+  // one call of run for both kinds of launch, so that its code is there once
   for (;;) {
-    // one queue pull per workgroup; the second barrier keeps the next pull
-    // from overwriting next_tile before every wave has read it
-    if (threadIdx.x == 0) next_tile = (int)atomicAdd(&L.queue[0], 1u);
-    __syncthreads();
-    const int tile = __builtin_amdgcn_readfirstlane(next_tile);
-    __syncthreads();
+    int tile = blockIdx.x;
+    if (L.grid > 0) {
+      // one queue pull per workgroup; the second barrier keeps the next pull
+      // from overwriting next_tile before every wave has read it
+      if (threadIdx.x == 0) next_tile = (int)atomicAdd(&L.queue[0], 1u);
+      __syncthreads();
+      tile = __builtin_amdgcn_readfirstlane(next_tile);
+      __syncthreads();
+    }
     if (tile >= ntiles) break;
     TT::run(L, tile, lds, lane, wave);
+    if (L.grid <= 0) return;
   }
+  if (L.grid <= 0) return;
   if (threadIdx.x == 0) {
     __threadfence();
     const unsigned fin = atomicAdd(&L.queue[1], 1u);
