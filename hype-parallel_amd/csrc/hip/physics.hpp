@@ -75,12 +75,11 @@ __device__ __forceinline__ double add_pressure(double a, double p) {
 struct Euler {
   static constexpr int NV = 4;
   static constexpr int WAVES_PER_EU = 2;  // register budget of the stage kernel: 256 per lane
-  // tile layouts the stage kernel is built for (bit 0: one wave per tile,
-  // bit 1: split tiles on two-wave workgroups); the host picks per problem.
-  // Split tiles run one wave per SIMD, one-wave tiles two: small grids gain
+  // tile layouts the stage kernel is built for (bit HYPE_LAYOUT_*: one wave per
+  // tile, split tiles, shared rows); the host picks per problem.  Split tiles run one wave per SIMD, one-wave tiles two: small grids gain
   // from the shorter sweeps (256^2: 540 -> 601 Mcell-updates/s), large ones
   // from the second wave's latency hiding
-  static constexpr int PAIR_MODES = 3;
+  static constexpr int PAIR_MODES = 7;
   // a split tile sends its CFL maximum to memory once, from the lower wave,
   // instead of once per wave: the atomics of the last stage contend for one
   // address (Euler quadrants 256^2: 636 -> 670 Mcell-updates/s)
@@ -202,7 +201,7 @@ struct Kapila {
   static constexpr int WAVES_PER_EU = 1;
   // split tiles only: one reconstructed ring row per wave saved at the same
   // one wave per SIMD (1024 x 512 shock-bubble: 952 -> 985 Mcell-updates/s)
-  static constexpr int PAIR_MODES = 2;
+  static constexpr int PAIR_MODES = 6;
   // one atomic per split tile (Kapila 1024x512: 1087 -> 1108
   // Mcell-updates/s; the batched set, whose 64 instances already spread the
   // atomics over 64 addresses, 1320 -> 1317)
@@ -465,7 +464,7 @@ struct BN {
   static constexpr int WAVES_PER_EU = 1;
   // one wave per tile only: two windows of nine components would halve the
   // workgroups an LDS of 160 KB holds
-  static constexpr int PAIR_MODES = 1;
+  static constexpr int PAIR_MODES = 5;
   static constexpr bool PAIR_CFL_COMBINE = false;  // one wave per tile
   static constexpr bool HAS_INLET = false;  // no InletBC in baer_nunziato.c
   // no sound speed is shared between the admissibility check and the flux

@@ -40,6 +40,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+#include <type_traits>
+
 #include "../../../include/hype2d.h"
 #include "../hype_internal.h"
 #include "physics.hpp"
@@ -182,6 +185,10 @@ __device__ __forceinline__ double lane_from_right(double v) {
                           __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false));
 }
 
+__device__ __forceinline__ int lane_from_left_int(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false);
+}
+
 // a value every lane computes alike, as a scalar
 __device__ __forceinline__ double uniform(double v) {
   return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
@@ -269,6 +276,25 @@ struct Tile {
       return r1_h * (F1 - F0 + 0.5 * (E1 + E0));
     else
       return (0.5 * Qd::WF * r1_h) * (F1 - F0 + (E1 + E0));
+  }
+
+  // add volume point q's product to the sum; its weight, a power of two, is
+  // applied once to the sum (+0 for a zero sum) unless terms may be subnormal
+  template <int q>
+  __device__ static __forceinline__ void add_volume(const double* B, double* ncp) {
+    static_for<NV>([&](auto c) {
+      if constexpr (S::DNZ[c]) {
+        if constexpr (S::JUMP_TINY[c])
+          ncp[c] = ncp[c] + -Qd::WV * B[c];
+        else
+          ncp[c] = q == 0 ? B[c] : ncp[c] + B[c];
+      }
+    });
+  }
+  __device__ static __forceinline__ void scale_volume(double* ncp) {
+    static_for<NV>([&](auto c) {
+      if constexpr (S::DNZ[c] && !S::JUMP_TINY[c]) ncp[c] = fma(-Qd::WV, ncp[c], 0.0);
+    });
   }
 
   // values of all components at the nodes, which are the face points
@@ -779,19 +805,9 @@ struct Tile {
             double V[NV], gx[NV], gy[NV], B[NV];
             at_vol<q>(co, r1_h, V, gx, gy);
             S::template vol_ncp<PRIM>(eos, V, gx, gy, B);
-#pragma unroll
-            for (int c = 0; c < NV; ++c)
-              if (S::DNZ[c]) {
-                if (S::JUMP_TINY[c])
-                  ncp[c] = ncp[c] + -Qd::WV * B[c];
-                else
-                  ncp[c] = q == 0 ? B[c] : ncp[c] + B[c];
-              }
+            add_volume<q>(B, ncp);
           });
-          // the weight, a power of two, once for the sum; +0 for a zero sum
-#pragma unroll
-          for (int c = 0; c < NV; ++c)
-            if (S::DNZ[c] && !S::JUMP_TINY[c]) ncp[c] = fma(-Qd::WV, ncp[c], 0.0);
+          scale_volume(ncp);
         }
       }
 
@@ -977,23 +993,31 @@ struct Tile {
   }
 };
 
-// Split tiles run one wave per SIMD: the two waves of a workgroup must not
-// share a SIMD's issue slots while other SIMDs idle.  A system whose kernel
+}  // namespace HYPE_KNS
+
+#include "duo.hpp"
+
+namespace HYPE_KNS {
+
+// Two-wave workgroups run one wave per SIMD: the two waves of a workgroup must
+// not share a SIMD's issue slots while other SIMDs idle.  A system whose kernel
 // would fit two waves per SIMD gets its accumulation registers reserved (an
 // empty asm statement that clobbers a255), which leaves room for one wave.
-template <class S, bool PR>
+template <class S, int LAY>
 struct Occ {
-  static constexpr bool ONE_PER_SIMD = PR && S::WAVES_PER_EU > 1;
-  static constexpr int WAVES_PER_EU = PR ? 1 : S::WAVES_PER_EU;
+  static constexpr bool ONE_PER_SIMD = LAY != HYPE_LAYOUT_ONE && S::WAVES_PER_EU > 1;
+  static constexpr int WAVES_PER_EU = LAY != HYPE_LAYOUT_ONE ? 1 : S::WAVES_PER_EU;
 };
+template <class S, bool PRIM, int N, int LAY, bool IN>
+using Body = std::conditional_t<LAY == HYPE_LAYOUT_DUO, Duo<S, PRIM, N, IN>, Tile<S, PRIM, N, LAY == HYPE_LAYOUT_SPLIT, IN>>;
 
 // IN: the build with the left-inlet ghost columns (Kapila problems with an
 // inlet only, so the loop of every other problem is compiled without it)
-template <class S, bool PRIM, int N, bool PR, bool IN>
-__global__ __launch_bounds__(PR ? 2 * HYPE_WAVE : HYPE_WAVE)
-    __attribute__((amdgpu_waves_per_eu(Occ<S, PR>::WAVES_PER_EU))) void stage_kernel(hype_launch L) {
-  using TT = Tile<S, PRIM, N, PR, IN>;
-  if constexpr (Occ<S, PR>::ONE_PER_SIMD) asm volatile("" ::: "a255");
+template <class S, bool PRIM, int N, int LAY, bool IN>
+__global__ __launch_bounds__(LAY ? 2 * HYPE_WAVE : HYPE_WAVE)
+    __attribute__((amdgpu_waves_per_eu(Occ<S, LAY>::WAVES_PER_EU))) void stage_kernel(hype_launch L) {
+  using TT = Body<S, PRIM, N, LAY, IN>;
+  if constexpr (Occ<S, LAY>::ONE_PER_SIMD) asm volatile("" ::: "a255");
   __shared__ double lds[TT::LDS];
   __shared__ int next_tile;
   const int lane = (int)threadIdx.x % HYPE_WAVE;
@@ -1025,32 +1049,47 @@ __global__ __launch_bounds__(PR ? 2 * HYPE_WAVE : HYPE_WAVE)
   }
 }
 
-template <class S, bool PRIM, int N, bool PR, bool IN>
+// layouts built for an order: shared rows only where the reconstruction is worth
+// sharing, and not with the 81 coefficients per lane of nine components at order
+// 3, whose LDS leaves one workgroup per CU (512x256: 1082 -> 1442 us per step)
+template <class S, int N>
+static constexpr int layouts() {
+#if defined(HYPE_CONTRACTED_BUILD)
+  return S::PAIR_MODES & 3;  // its solves use the layouts of batches (hype_layouts)
+#else
+  return N == 2 || (N == 3 && S::NV <= 6) ? S::PAIR_MODES : S::PAIR_MODES & 3;
+#endif
+}
+
+template <class S, bool PRIM, int N, int LAY, bool IN>
 static hipError_t launch_variant(const hype_launch& L, hipStream_t s) {
   // one workgroup per table entry (grid 0; with a device-resident count the
   // workgroups past it return at once), or a persistent grid pulling tiles
   const int grid = L.grid > 0 ? L.grid : L.ntiles;
-  hipLaunchKernelGGL((stage_kernel<S, PRIM, N, PR, IN>), dim3(grid), dim3(HYPE_WAVE * Tile<S, PRIM, N, PR, IN>::WAVES), 0,
+  hipLaunchKernelGGL((stage_kernel<S, PRIM, N, LAY, IN>), dim3(grid), dim3(HYPE_WAVE * Body<S, PRIM, N, LAY, IN>::WAVES), 0,
                      s, L);
   return hipGetLastError();
 }
 
-template <class S, bool PRIM, int N, bool PR>
+template <class S, bool PRIM, int N, int LAY>
 static hipError_t launch_inlet(const hype_launch& L, hipStream_t s) {
   if (L.v.inlet) {
-    if constexpr (S::HAS_INLET) return launch_variant<S, PRIM, N, PR, true>(L, s);
+    if constexpr (S::HAS_INLET) return launch_variant<S, PRIM, N, LAY, true>(L, s);
     return hipErrorInvalidValue;
   }
-  return launch_variant<S, PRIM, N, PR, false>(L, s);
+  return launch_variant<S, PRIM, N, LAY, false>(L, s);
 }
 
 // the tile layout the variant asks for, if the system is built for it
 template <class S, bool PRIM, int N>
 static hipError_t launch_layout(const hype_launch& L, hipStream_t s) {
-  if (L.v.pair) {
-    if constexpr ((S::PAIR_MODES & 2) != 0) return launch_inlet<S, PRIM, N, true>(L, s);
+  constexpr int modes = layouts<S, N>();
+  if (L.v.pair == HYPE_LAYOUT_DUO) {
+    if constexpr ((modes & 4) != 0) return launch_inlet<S, PRIM, N, HYPE_LAYOUT_DUO>(L, s);
+  } else if (L.v.pair == HYPE_LAYOUT_SPLIT) {
+    if constexpr ((modes & 2) != 0) return launch_inlet<S, PRIM, N, HYPE_LAYOUT_SPLIT>(L, s);
   } else {
-    if constexpr ((S::PAIR_MODES & 1) != 0) return launch_inlet<S, PRIM, N, false>(L, s);
+    if constexpr ((modes & 1) != 0) return launch_inlet<S, PRIM, N, HYPE_LAYOUT_ONE>(L, s);
   }
   return hipErrorInvalidValue;
 }
@@ -1066,30 +1105,37 @@ static hipError_t launch_sys(const hype_launch& L, hipStream_t s) {
   }
 }
 
-template <class S, bool PRIM, int N, bool PR, bool IN>
+template <class S, bool PRIM, int N, int LAY, bool IN>
 static int occupancy_variant() {
-  int blocks = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, stage_kernel<S, PRIM, N, PR, IN>,
-                                                   HYPE_WAVE * Tile<S, PRIM, N, PR, IN>::WAVES, 0) != hipSuccess)
+  // a property of the compiled kernel, asked of the runtime once (about 30 us)
+  static std::atomic<int> known{-1};
+  int blocks = known.load(std::memory_order_relaxed);
+  if (blocks >= 0) return blocks;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, stage_kernel<S, PRIM, N, LAY, IN>,
+                                                   HYPE_WAVE * Body<S, PRIM, N, LAY, IN>::WAVES, 0) != hipSuccess)
     return 0;
+  known.store(blocks, std::memory_order_relaxed);
   return blocks;
 }
 
-template <class S, bool PRIM, int N, bool PR>
+template <class S, bool PRIM, int N, int LAY>
 static int occupancy_inlet(const hype_variant& v) {
   if (v.inlet) {
-    if constexpr (S::HAS_INLET) return occupancy_variant<S, PRIM, N, PR, true>();
+    if constexpr (S::HAS_INLET) return occupancy_variant<S, PRIM, N, LAY, true>();
     return 0;
   }
-  return occupancy_variant<S, PRIM, N, PR, false>();
+  return occupancy_variant<S, PRIM, N, LAY, false>();
 }
 
 template <class S, bool PRIM, int N>
 static int occupancy_layout(const hype_variant& v) {
-  if (v.pair) {
-    if constexpr ((S::PAIR_MODES & 2) != 0) return occupancy_inlet<S, PRIM, N, true>(v);
+  constexpr int modes = layouts<S, N>();
+  if (v.pair == HYPE_LAYOUT_DUO) {
+    if constexpr ((modes & 4) != 0) return occupancy_inlet<S, PRIM, N, HYPE_LAYOUT_DUO>(v);
+  } else if (v.pair == HYPE_LAYOUT_SPLIT) {
+    if constexpr ((modes & 2) != 0) return occupancy_inlet<S, PRIM, N, HYPE_LAYOUT_SPLIT>(v);
   } else {
-    if constexpr ((S::PAIR_MODES & 1) != 0) return occupancy_inlet<S, PRIM, N, false>(v);
+    if constexpr ((modes & 1) != 0) return occupancy_inlet<S, PRIM, N, HYPE_LAYOUT_ONE>(v);
   }
   return 0;
 }
@@ -1115,13 +1161,17 @@ hipError_t launch_stage_bn(const hype_launch& L, hipStream_t s);
 int blocks_per_cu_bn(const hype_variant& v);
 #endif
 
-// tile layouts a system's stage kernel is built for (bit 0: one wave per
-// tile, bit 1: split tiles)
-int pair_modes(int system) {
+// tile layouts a system's stage kernel of an order is built for (bit
+// HYPE_LAYOUT_*)
+template <class S>
+static int layouts_of(int order) {
+  return order == 0 ? layouts<S, 0>() : order == 1 ? layouts<S, 1>() : order == 2 ? layouts<S, 2>() : layouts<S, 3>();
+}
+int pair_modes(int system, int order) {
   switch (system) {
-    case HYPE_EULER: return Euler::PAIR_MODES;
-    case HYPE_KAPILA: return Kapila::PAIR_MODES;
-    default: return BN::PAIR_MODES;
+    case HYPE_EULER: return layouts_of<Euler>(order);
+    case HYPE_KAPILA: return layouts_of<Kapila>(order);
+    default: return layouts_of<BN>(order);
   }
 }
 

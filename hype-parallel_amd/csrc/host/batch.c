@@ -240,7 +240,7 @@ int hype_batch_autotune(hype_batch *b, const int *cand, int ncand, int steps, in
     int *maxs;
     if (!b || !cand || ncand < 1 || steps < 1) return HYPE_E_INVALID;
     for (i = 0; i < b->n; ++i)
-        if (hype_layouts(&b->E.P[i], hyped_pair_modes(b->E.P[i].system)) == 3) nlay = 2;
+        if ((hype_layouts(&b->E.P[i], hyped_pair_modes(b->E.P[i].system, b->E.P[i].order)) & 3) == 3) nlay = 2;
     t_end = (double *)malloc((size_t)b->n * sizeof(double));
     maxs = (int *)malloc((size_t)b->n * sizeof(int));
     if (!t_end || !maxs) {

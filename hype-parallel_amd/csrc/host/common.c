@@ -73,7 +73,9 @@ int hype_strips(int nx) { return (nx + HYPE_TILE_W - 1) / HYPE_TILE_W; }
  * about (h + 2 + c0) row-iterations (two ring rows, c0 for the 5-row
  * prologue).  Where the two halves of a tile run on two waves (pair), each
  * wave sweeps about h/2 rows plus one ring row, and the two meet at one
- * face (a quarter of an iteration).  The kernel is bound by FP64 issue:
+ * face (a quarter of an iteration).  Where they share every row (pair =
+ * HYPE_LAYOUT_DUO), each takes about 0.54 of every row, ring rows included.  The
+ * kernel is bound by FP64 issue:
  * waves that share a SIMD share its issue slots, gaining only latency
  * hiding (a measured 1.5x for two waves).  With w = ceil(waves / simds)
  * waves per SIMD and `occ` resident waves per SIMD, a launch therefore takes
@@ -86,8 +88,20 @@ static double occ_gain(long w) { return w >= 2 ? 1.5 : 1.0; }
 double hype_tile_rows(int h, int pair)
 {
     const double c0 = 1.0;
+    if (pair == HYPE_LAYOUT_DUO) return 0.54 * (h + 2.0) + c0;
     if (pair && h >= 2) return (double)((h + 1) / 2) + 1.0 + c0 + 0.25;
     return h + 2.0 + c0;
+}
+
+/* Row-iterations of a wave for a tile of h rows whose rows two waves share.
+ * The share of a row that one wave takes was measured on grids of one round of
+ * tiles, from the time each further row adds: Euler 2.85 of 4.87 us, Kapila 4.87
+ * of 9.0 us, Baer-Nunziato 7.9 of 16.3 us (conservative path) and 7.5 of 13.1 us
+ * (primitive path). */
+static double duo_rows(const hype_problem *p, int h)
+{
+    const double share = p->system == HYPE_EULER ? 0.585 : p->system == HYPE_KAPILA ? 0.54 : p->recons_prim ? 0.57 : 0.49;
+    return share * (h + 2.0) + 1.0;
 }
 
 double hype_tile_cost(long waves, double per, int simds, int occ)
@@ -158,13 +172,15 @@ void hype_decode_error(unsigned long long word, int nx, int ny, int ngf,
     snprintf(msg, cap, "%s\nAt x = %f, y = %f", head, *x, *y);
 }
 
-/* tile layouts (bit 0: one wave per tile, bit 1: split tiles) a problem may
- * use: those the system's kernel is built for, narrowed by the layout bits
+/* tile layouts (bits HYPE_LAYOUT_*) a problem may use: those the system's kernel is built for, narrowed by the layout bits
  * of its options */
 int hype_layouts(const hype_problem *p, int built)
 {
     if (p->options & HYPE_OPT_ONE_WAVE_TILES) return built & 1;
     if (p->options & HYPE_OPT_SPLIT_TILES) return built & 2;
+    /* contraction differs between the layouts' kernels: a contracted solve keeps
+     * to those of batches and servers, whose results it must match */
+    if (p->options & HYPE_OPT_FMA) return built & 3;
     return built;
 }
 
@@ -242,13 +258,13 @@ int hype_xcd_order(hype_tile *tiles, int n, int nxcd)
 
 int hype_pick_layout(const hype_problem *p, int *pair, int *nsy, int *slots)
 {
-    const int modes = hype_layouts(p, hyped_pair_modes(p->system));
+    const int modes = hype_layouts(p, hyped_pair_modes(p->system, p->order));
     int ncu = hyped_num_cus(), pr, found = 0;
     double best = 1e300;
     if (ncu < 1) ncu = 256;
-    for (pr = 0; pr <= 1; ++pr) {
+    for (pr = HYPE_LAYOUT_ONE; pr <= HYPE_LAYOUT_DUO; ++pr) {
         hype_variant v;
-        int sl, occ, ns;
+        int sl, occ, ns, h;
         double cost;
         if (!(modes & (1 << pr))) continue;
         v.system = p->system;
@@ -261,8 +277,9 @@ int hype_pick_layout(const hype_problem *p, int *pair, int *nsy, int *slots)
         if (sl < 1) sl = 4 * ncu;
         occ = (sl + 4 * ncu - 1) / (4 * ncu);
         ns = hype_pick_segments(p->nx, p->ny, 4 * ncu, occ, 0, pr);
+        h = (p->ny + ns - 1) / ns;
         cost = hype_tile_cost((long)hype_strips(p->nx) * ns * hyped_block_waves(&v),
-                              hype_tile_rows((p->ny + ns - 1) / ns, pr), 4 * ncu, occ);
+                              pr == HYPE_LAYOUT_DUO ? duo_rows(p, h) : hype_tile_rows(h, pr), 4 * ncu, occ);
         if (cost < best - 1e-9) {
             best = cost;
             *pair = pr;

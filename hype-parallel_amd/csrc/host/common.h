@@ -26,11 +26,10 @@ int hype_pick_segments(int nx, int ny, int simds, int occ, int extra_waves, int 
  * or conserved as the problem's path stores ghost cells */
 size_t hype_inlet_doubles(const hype_problem *p);
 void hype_inlet_table(const hype_problem *p, double *out);
-/* tile layouts a problem may use (bit 0: one wave per tile, bit 1: split
- * tiles), given those its system's kernel is built for */
+/* tile layouts a problem may use (bits HYPE_LAYOUT_*), given those its system's
+ * kernel is built for */
 int hype_layouts(const hype_problem *p, int built);
-/* tile layout (*pair: 1 split tiles on two-wave workgroups, 0 one wave per
- * tile) and row segments of a single grid: the tile-shape model's cheapest
+/* tile layout (*pair: HYPE_LAYOUT_*) and row segments of a single grid: the tile-shape model's cheapest
  * among the layouts the system's kernel is built for; *slots (may be NULL)
  * receives the resident waves of that kernel on the device */
 int hype_pick_layout(const hype_problem *p, int *pair, int *nsy, int *slots);

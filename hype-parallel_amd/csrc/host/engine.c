@@ -128,7 +128,7 @@ static int find_group(hype_engine *E, const hype_variant *v)
 /* the kernel variant of a problem in this engine */
 static int slot_variant(const hype_engine *E, const hype_problem *p, hype_variant *v)
 {
-    const int modes = hype_layouts(p, hyped_pair_modes(p->system));
+    const int modes = hype_layouts(p, hyped_pair_modes(p->system, p->order));
     if (!modes) return HYPE_E_UNSUPPORTED;
     v->system = p->system;
     v->prim = p->recons_prim;
@@ -138,8 +138,8 @@ static int slot_variant(const hype_engine *E, const hype_problem *p, hype_varian
      * for them), or where both are built and the engine prefers them; by
      * default a batch keeps many waves per SIMD busy, where one-wave tiles
      * hide latency better */
-    if (modes == 3 && E->layout >= 0) v->pair = E->layout;
-    else v->pair = (modes & 1) ? 0 : 1;
+    if ((modes & 3) == 3 && E->layout >= 0) v->pair = E->layout;
+    else v->pair = (modes & 1) ? HYPE_LAYOUT_ONE : HYPE_LAYOUT_SPLIT;
     v->inlet = p->bc[0] == HYPE_BC_INLET;
     return HYPE_OK;
 }

@@ -81,11 +81,18 @@ typedef struct hype_tile {
 #define HYPE_MODE_RHS 1
 #define HYPE_MODE_PRIME 2
 
+/* tile layouts of the stage kernel: one wave per tile; a tile split at its
+ * middle row over the two waves of a workgroup; both waves of a workgroup on
+ * every row of its tile */
+#define HYPE_LAYOUT_ONE 0
+#define HYPE_LAYOUT_SPLIT 1
+#define HYPE_LAYOUT_DUO 2
+
 /* kernel variant: system x path x order */
 typedef struct hype_variant {
     int system, prim, order;
     int fma;               /* 1: the FMA-contracted kernel build (HYPE_OPT_FMA) */
-    int pair;              /* 1: each tile split over a two-wave workgroup */
+    int pair;              /* HYPE_LAYOUT_* */
     int inlet;             /* 1: the build with left-inlet ghost columns */
 } hype_variant;
 
@@ -144,12 +151,11 @@ int hyped_mem_info(size_t *free_bytes, size_t *total_bytes);
 int hyped_num_cus(void);
 /* resident workgroups per CU of the stage kernel of a variant */
 int hyped_blocks_per_cu(const hype_variant *v);
-/* waves per workgroup of that kernel: 2 with split tiles (the two halves of
- * each tile on their own waves, see the stage kernel), else 1 */
+/* waves per workgroup of that kernel: 1 with one wave per tile, else 2 */
 int hyped_block_waves(const hype_variant *v);
-/* tile layouts a system's stage kernel is built for: bit 0 one wave per
- * tile, bit 1 split tiles */
-int hyped_pair_modes(int system);
+/* tile layouts (bits HYPE_LAYOUT_*) a system's stage kernel of an order is built
+ * for */
+int hyped_pair_modes(int system, int order);
 const char *hyped_last_error(void);
 /* this device's address of the scratch array and its size (looked up on the
  * first call on each device, with that device current) */

@@ -89,10 +89,11 @@ typedef struct hype_problem {
 #define HYPE_OPT_FMA 0x1u
 
 /* ---- tile layout ----------------------------------------------------------
- * The stage kernel sweeps tiles of up to 62 columns.  A tile runs either on
- * one wave, or split at its middle row over the two waves of a workgroup,
- * which saves one reconstructed ring row per wave.  By default
- * hype_ctx_create picks the faster layout for the grid (Kapila: split;
+ * The stage kernel sweeps tiles of up to 62 columns.  A tile runs on one
+ * wave, or split at its middle row over the two waves of a workgroup, which
+ * saves one reconstructed ring row per wave, or with both waves sharing the
+ * work of every row.  By default hype_ctx_create picks the faster layout for
+ * the grid (shared rows for tiles a few rows high; otherwise Kapila: split;
  * Baer-Nunziato: one wave; Euler: split for small grids, one wave when the
  * grid fills two waves per SIMD), and batches and servers use split tiles
  * for Kapila and one wave per tile otherwise.  These bits force a layout; one
