@@ -69,7 +69,7 @@ int hyped_free(void* p) {
 int hyped_host_alloc(void** p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) bytes = 8;
-  hipError_t e = hipHostMalloc(p, bytes, hipHostMallocDefault);
+  hipError_t e = hipHostMalloc(p, bytes, hipHostMallocPortable);
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
     snprintf(g_err, sizeof(g_err), "hipHostMalloc(%zu): out of memory", bytes);

@@ -603,18 +603,10 @@ struct Duo {
       const double m = wave_max((wave == 0 ? xlane : owned) ? smax : 0.0);
       if (wave == 1 && lane == 0) *y_smax = m;
       __syncthreads();
-      if (wave == 0 && lane == 0) {
-        unsigned long long* slotp =
-            (mode == HYPE_MODE_RHS) ? &st->smax_rhs : (mode == HYPE_MODE_PRIME ? &st->smax[st->step & 1] : &st->smax[(cur + 1) & 1]);
-        atomicMax(slotp, (unsigned long long)__double_as_longlong(fmax(m, *y_smax)));
-      }
+      if (wave == 0 && lane == 0) send_smax(L, st, cur, fmax(m, *y_smax));
     }
     const unsigned long long e = wave_min_u64(err);
-    if (lane == 0 && e != ~0ull) {
-      unsigned long long* ep =
-          (mode == HYPE_MODE_RHS) ? &st->err_rhs : (mode == HYPE_MODE_PRIME ? &st->err[1] : &st->err[cur & 1]);
-      atomicMin(ep, e);
-    }
+    if (lane == 0) send_error(L, st, cur, e);
   }
 };
 

@@ -8,6 +8,8 @@
  * during a solve: the last stage of every step reduces the wave speed on the
  * device and the first stage of the next step turns it into dt.
  */
+#include <pthread.h>
+#include <stddef.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -22,10 +24,12 @@ struct hype_ctx {
     void *stream;
     double *buf[3];         /* U, A, B (device) */
     double *R;              /* RHS output (device) */
-    hype_dstate *st;        /* device time state */
+    hype_dstate *st;        /* device time state; the descriptor and the queue
+                               counters share its allocation */
     hype_inst *inst_d;
     hype_tile *tiles_d;
     unsigned *queue_d;
+    struct ctx_host *host;  /* pinned host memory the device reports into */
     double *hist_d;
     int hist_cap;
     unsigned char *fb_d;
@@ -38,6 +42,86 @@ struct hype_ctx {
     double err_x, err_y;
 };
 
+struct ctx_host {
+    unsigned long long rhs[2]; /* smax_rhs, err_rhs of the last RHS evaluation */
+    hype_dstate st;            /* time state as of the last hype_sync */
+};
+
+/* Pinned slots for the contexts' host structs.  Pinning a page takes longer than
+ * the rest of hype_ctx_create (about 160 us), so contexts share pages of
+ * CTX_SLOTS slots; a page is returned when its last slot is, unless it is the only
+ * one left: at most one empty page (8 KB) stays with the process.  Any thread. */
+#define CTX_SLOTS 32
+#define CTX_SLOT_BYTES 256
+typedef struct host_page {
+    struct host_page *next;
+    unsigned char *mem;
+    unsigned used; /* bit per slot */
+} host_page;
+static pthread_mutex_t host_mu = PTHREAD_MUTEX_INITIALIZER;
+static host_page *host_pages;
+
+static int host_acquire(struct ctx_host **out)
+{
+    host_page *p;
+    int k, rc = HYPE_OK;
+    _Static_assert(sizeof(struct ctx_host) <= CTX_SLOT_BYTES, "a slot holds a context's host struct");
+    *out = NULL;
+    pthread_mutex_lock(&host_mu);
+    for (p = host_pages; p && p->used == ~0u; p = p->next) {
+    }
+    if (!p) {
+        p = (host_page *)calloc(1, sizeof(*p));
+        rc = p ? hyped_host_alloc((void **)&p->mem, CTX_SLOTS * CTX_SLOT_BYTES) : HYPE_E_NOMEM;
+        if (rc == HYPE_OK) {
+            p->next = host_pages;
+            host_pages = p;
+        } else {
+            free(p);
+        }
+    }
+    if (rc == HYPE_OK) {
+        for (k = 0; p->used & (1u << k); ++k) {
+        }
+        p->used |= 1u << k;
+        *out = (struct ctx_host *)(p->mem + k * CTX_SLOT_BYTES);
+    }
+    pthread_mutex_unlock(&host_mu);
+    return rc;
+}
+
+static void host_release(struct ctx_host *h)
+{
+    host_page **pp, *p;
+    if (!h) return;
+    pthread_mutex_lock(&host_mu);
+    for (pp = &host_pages; (p = *pp) != NULL; pp = &p->next) {
+        const ptrdiff_t off = (unsigned char *)h - p->mem;
+        if (off < 0 || off >= CTX_SLOTS * CTX_SLOT_BYTES) continue;
+        p->used &= ~(1u << (off / CTX_SLOT_BYTES));
+        if (p->used == 0 && (p != host_pages || p->next)) {
+            *pp = p->next;
+            hyped_host_free(p->mem);
+            free(p);
+        }
+        break;
+    }
+    pthread_mutex_unlock(&host_mu);
+}
+
+/* offsets in the allocation of the time state */
+#define CTX_INST_OFF 256
+#define CTX_QUEUE_OFF 512
+#define CTX_SMALL_BYTES 768
+
+static void init_state(hype_dstate *d)
+{
+    memset(d, 0, sizeof(*d));
+    d->err[0] = ~0ull;
+    d->err[1] = ~0ull;
+    d->err_rhs = ~0ull;
+}
+
 static void ctx_free(hype_ctx *c)
 {
     int i;
@@ -46,9 +130,8 @@ static void ctx_free(hype_ctx *c)
     for (i = 0; i < 3; ++i) hyped_free(c->buf[i]);
     hyped_free(c->R);
     hyped_free(c->st);
-    hyped_free(c->inst_d);
+    host_release(c->host);
     hyped_free(c->tiles_d);
-    hyped_free(c->queue_d);
     hyped_free(c->hist_d);
     hyped_free(c->fb_d);
     hyped_free(c->inlet_d);
@@ -61,6 +144,9 @@ int hype_ctx_create(const hype_problem *p, hype_ctx **out)
     hype_ctx *c;
     hype_tile *tiles;
     int rc, nv = 0, i;
+    _Alignas(16) unsigned char small[CTX_SMALL_BYTES];
+    _Static_assert(sizeof(hype_dstate) <= CTX_INST_OFF, "time state overlaps the descriptor");
+    _Static_assert(CTX_INST_OFF + sizeof(hype_inst) <= CTX_QUEUE_OFF, "descriptor overlaps the queue");
     if (!out) return HYPE_E_INVALID;
     *out = NULL;
     HYPE_TRY(hype_check_problem(p, &nv));
@@ -84,11 +170,11 @@ int hype_ctx_create(const hype_problem *p, hype_ctx **out)
     for (i = 0; i < 3; ++i)
         if ((rc = hyped_malloc((void **)&c->buf[i], c->nbytes)) != HYPE_OK) goto fail;
     if ((rc = hyped_malloc((void **)&c->R, c->nbytes)) != HYPE_OK) goto fail;
-    if ((rc = hyped_malloc((void **)&c->st, sizeof(hype_dstate))) != HYPE_OK) goto fail;
-    if ((rc = hyped_malloc((void **)&c->inst_d, sizeof(hype_inst))) != HYPE_OK) goto fail;
+    if ((rc = hyped_malloc((void **)&c->st, CTX_SMALL_BYTES)) != HYPE_OK) goto fail;
+    c->inst_d = (hype_inst *)((char *)c->st + CTX_INST_OFF);
+    c->queue_d = (unsigned *)((char *)c->st + CTX_QUEUE_OFF);
+    if ((rc = host_acquire(&c->host)) != HYPE_OK) goto fail;
     if ((rc = hyped_malloc((void **)&c->tiles_d, (size_t)c->ntiles * sizeof(hype_tile))) != HYPE_OK) goto fail;
-    if ((rc = hyped_malloc((void **)&c->queue_d, 4 * sizeof(unsigned))) != HYPE_OK) goto fail;
-    if ((rc = hyped_fill_u64(c->queue_d, 0ull, 2, c->stream)) != HYPE_OK) goto fail;
 
     hype_fill_inst(&c->inst_h, p, c->nsy);
     c->inst_h.buf[0] = c->buf[0];
@@ -108,7 +194,11 @@ int hype_ctx_create(const hype_problem *p, hype_ctx **out)
         if (rc != HYPE_OK) goto fail;
         c->inst_h.inlet = c->inlet_d;
     }
-    if ((rc = hyped_memcpy_h2d(c->inst_d, &c->inst_h, sizeof(hype_inst), c->stream)) != HYPE_OK) goto fail;
+    /* time state, descriptor and zeroed queue counters in one copy */
+    memset(small, 0, sizeof(small));
+    init_state((hype_dstate *)small);
+    memcpy(small + CTX_INST_OFF, &c->inst_h, sizeof(hype_inst));
+    if ((rc = hyped_memcpy_h2d(c->st, small, sizeof(small), c->stream)) != HYPE_OK) goto fail;
     tiles = (hype_tile *)malloc((size_t)c->ntiles * sizeof(hype_tile));
     if (!tiles) { rc = HYPE_E_NOMEM; goto fail; }
     if (hype_make_tiles(0, p->nx, p->ny, hype_strips(p->nx), c->nsy, tiles, c->ntiles) != c->ntiles)
@@ -169,7 +259,6 @@ const char *hype_last_error(hype_ctx *c, double *x, double *y)
 static int rhs_impl(hype_ctx *c, const double *U, double *RHS, double *dt_out,
                     unsigned char *fallback, int mem)
 {
-    unsigned long long slots[2] = {0ull, ~0ull}; /* smax_rhs, err_rhs */
     const double *in;
     double *out;
     hype_launch L;
@@ -182,10 +271,12 @@ static int rhs_impl(hype_ctx *c, const double *U, double *RHS, double *dt_out,
         in = U;
         out = RHS;
     }
-    HYPE_TRY(hyped_memcpy_h2d(&c->st->smax_rhs, slots, sizeof(slots), c->stream));
+    /* the last tile writes the maximum and the error word to c->host and leaves
+     * the slots reset, so nothing is copied before or after the launch */
     L = base_launch(c, HYPE_MODE_RHS, 0);
     L.rhs_in = in;
     L.rhs_out = out;
+    L.report = c->host->rhs;
     if (fallback) {
         if (!c->fb_d) HYPE_TRY(hyped_malloc((void **)&c->fb_d, c->ncell));
         L.fallback = c->fb_d;
@@ -193,14 +284,13 @@ static int rhs_impl(hype_ctx *c, const double *U, double *RHS, double *dt_out,
     HYPE_TRY(hyped_launch(&L, c->stream));
     if (mem == HYPE_MEM_HOST) HYPE_TRY(hyped_memcpy_d2h(RHS, c->R, c->nbytes, c->stream));
     if (fallback) HYPE_TRY(hyped_memcpy_d2h(fallback, c->fb_d, c->ncell, c->stream));
-    HYPE_TRY(hyped_memcpy_d2h(slots, &c->st->smax_rhs, sizeof(slots), c->stream));
     HYPE_TRY(hyped_stream_sync(c->stream));
     if (dt_out) {
         double smax, h = (c->P.x_max - c->P.x_min) / (double)(c->P.nx);
-        memcpy(&smax, &slots[0], sizeof(smax));
+        memcpy(&smax, &c->host->rhs[0], sizeof(smax));
         *dt_out = (c->P.cfl * h) / (2.0 * smax); /* rhs_function_prim.c:620 */
     }
-    if (slots[1] != ~0ull) return set_error(c, slots[1]);
+    if (c->host->rhs[1] != ~0ull) return set_error(c, c->host->rhs[1]);
     return HYPE_OK;
 }
 
@@ -274,20 +364,10 @@ int hype_begin(hype_ctx *c, double t0, double t_end, int max_steps, unsigned fla
             c->hist_cap = max_steps;
         }
     }
-    memset(&d, 0, sizeof(d));
+    init_state(&d);
     d.t = t0;
-    d.dt = 0.0;
     d.t_end = t_end;
-    d.smax[0] = 0ull;
-    d.smax[1] = 0ull;
-    d.smax_rhs = 0ull;
-    d.err[0] = ~0ull;
-    d.err[1] = ~0ull;
-    d.err_rhs = ~0ull;
-    d.step = 0;
-    d.cur = 0;
     d.max_steps = max_steps;
-    d.done = 0;
     d.clip = (flags & HYPE_TS_CLIP) ? 1 : 0;
     d.hist_len = c->hist_cap;
     d.dt_hist = c->hist_d;
@@ -347,8 +427,9 @@ int hype_sync(hype_ctx *c, hype_status *st)
     hype_dstate d;
     if (!c) return HYPE_E_INVALID;
     unsigned long long e;
-    HYPE_TRY(hyped_memcpy_d2h(&d, c->st, sizeof(d), c->stream));
+    HYPE_TRY(hyped_memcpy_d2h(&c->host->st, c->st, sizeof(d), c->stream));
     HYPE_TRY(hyped_stream_sync(c->stream));
+    d = c->host->st;
     /* the failing step is the last one taken (stepping stops after it);
      * with no step taken, a failure belongs to the priming call */
     e = d.step > 0 ? d.err[(d.step - 1) & 1] : d.err[1];

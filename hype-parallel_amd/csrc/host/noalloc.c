@@ -19,11 +19,12 @@
 #include "common.h"
 
 static pthread_mutex_t na_mu = PTHREAD_MUTEX_INITIALIZER;
-/* host staging of one call: descriptor and time state, tile table (model
- * order, then XCD order), inlet table */
-static unsigned char na_head[HYPE_SCRATCH_TILES_OFF];
+/* host staging of one call, laid out as the scratch up to the end of its tile
+ * table (descriptor, time state, tiles in XCD order), which one copy fills; the
+ * tiles in model order; the inlet table */
+static _Alignas(16) unsigned char na_head[HYPE_SCRATCH_INLET_OFF];
 static hype_tile na_rows[HYPE_SCRATCH_MAX_TILES];
-static hype_tile na_tiles[HYPE_SCRATCH_MAX_TILES];
+#define na_tiles ((hype_tile *)(na_head + HYPE_SCRATCH_TILES_OFF))
 static double na_inlet[HYPE_SCRATCH_INLET_DOUBLES];
 
 static int rhs_noalloc_locked(const hype_problem *p, const double *U, double *RHS, double *dt_out,
@@ -65,15 +66,13 @@ static int rhs_noalloc_locked(const hype_problem *p, const double *U, double *RH
     st.smax_rhs = 0ull;
     st.err_rhs = ~0ull;
     st.err[0] = st.err[1] = ~0ull;
-    memset(na_head, 0, sizeof(na_head));
+    memset(na_head, 0, HYPE_SCRATCH_TILES_OFF);
     memcpy(na_head, &inst, sizeof(inst));
     memcpy(na_head + HYPE_SCRATCH_STATE_OFF, &st, sizeof(st));
 
     /* from here on a failure waits for the stream before it returns, so
      * no copy out of the static staging is still pending for the next call */
-    rc = hyped_memcpy_h2d(base, na_head, sizeof(na_head), stream);
-    if (rc == HYPE_OK)
-        rc = hyped_memcpy_h2d(base + HYPE_SCRATCH_TILES_OFF, na_tiles, (size_t)ntiles * sizeof(hype_tile), stream);
+    rc = hyped_memcpy_h2d(base, na_head, HYPE_SCRATCH_TILES_OFF + (size_t)ntiles * sizeof(hype_tile), stream);
     if (rc == HYPE_OK && ninlet > 0)
         rc = hyped_memcpy_h2d(base + HYPE_SCRATCH_INLET_OFF, na_inlet, ninlet * sizeof(double), stream);
 

@@ -41,6 +41,8 @@ typedef struct hype_dstate {
     int clip;
     int hist_len;
     double *dt_hist;       /* optional: dt of every step */
+    unsigned rhs_done;     /* workgroup tiles finished by a reported RHS evaluation */
+    int pad1;
 } hype_dstate;
 
 /* per-instance descriptor read by the kernels */
@@ -110,6 +112,9 @@ typedef struct hype_launch {
     const double *rhs_in;      /* RHS/PRIME mode: input state override */
     double *rhs_out;           /* RHS mode: output */
     unsigned char *fallback;   /* RHS mode: optional per-cell fallback mask */
+    unsigned long long *report; /* RHS mode: pinned host words {smax_rhs, err_rhs}
+                                   the last tile writes, resetting the slots
+                                   for the next evaluation; or NULL */
 } hype_launch;
 
 /* device scratch of the allocation-free RHS (hype_rhs_noalloc, scratch.hip):
