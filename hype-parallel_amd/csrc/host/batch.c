@@ -101,7 +101,7 @@ int hype_batch_create(const hype_problem *probs, int n, const hype_batch_opts *o
             return rc;
         }
     }
-    if (b->opts.tile_rows < 1) eng_set_rows(&b->E, eng_pick_rows(&b->E));
+    if (b->opts.tile_rows < 1) eng_auto_rows(&b->E);
     if ((rc = eng_commit(&b->E)) != HYPE_OK) {
         hype_batch_destroy(b);
         return rc;

@@ -104,6 +104,14 @@ static double duo_rows(const hype_problem *p, int h)
     return share * (h + 2.0) + 1.0;
 }
 
+/* Time a wave takes for one row of a strip, in us: measured at order 2; order 3
+ * takes about 1.3 times, orders 0 and 1 a third of that. */
+double hype_row_time(const hype_problem *p)
+{
+    const double t = p->system == HYPE_EULER ? 4.87 : p->system == HYPE_KAPILA ? 9.0 : p->recons_prim ? 13.1 : 16.3;
+    return t * (p->order == 3 ? 1.3 : p->order == 2 ? 1.0 : 0.35);
+}
+
 double hype_tile_cost(long waves, double per, int simds, int occ)
 {
     long w;

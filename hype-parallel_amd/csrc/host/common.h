@@ -35,6 +35,8 @@ int hype_layouts(const hype_problem *p, int built);
 int hype_pick_layout(const hype_problem *p, int *pair, int *nsy, int *slots);
 /* row-iterations of one wave for a tile of h rows */
 double hype_tile_rows(int h, int pair);
+/* time of one row of a strip on one wave, in us */
+double hype_row_time(const hype_problem *p);
 /* modelled time of a launch of `waves` waves of `per` row-iterations each */
 double hype_tile_cost(long waves, double per, int simds, int occ);
 

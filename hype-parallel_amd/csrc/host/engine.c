@@ -203,13 +203,31 @@ int eng_set_running(hype_engine *E, int slot, int on)
     return HYPE_OK;
 }
 
-static int rows_for(const hype_engine *E, int slot)
+/* time a tile of a slot takes per row: a wave's row, of which each wave of a split
+ * tile takes every other one */
+static double tile_row_time(const hype_engine *E, int slot)
 {
-    int ny = E->P[slot].ny, h = E->target_rows > 0 ? E->target_rows : 16;
-    int nsy = (ny + h - 1) / h;
+    const int split = E->g[E->group_of[slot]].bwaves > 1;
+    return hype_row_time(&E->P[slot]) / (split ? 2.0 : 1.0);
+}
+
+/* row segments of a slot at a target height (weighted: scaled by its row time) */
+static int rows_at(const hype_engine *E, int slot, int target, int weighted, double row_min)
+{
+    int ny = E->P[slot].ny, h = target > 0 ? target : 16, nsy;
+    if (weighted) {
+        h = (int)(h * row_min / tile_row_time(E, slot));
+        if (h < 1) h = 1;
+    }
+    nsy = (ny + h - 1) / h;
     if (nsy < 1) nsy = 1;
     if (nsy > ny) nsy = ny;
     return nsy;
+}
+
+static int rows_for(const hype_engine *E, int slot)
+{
+    return rows_at(E, slot, E->target_rows, E->weighted, E->row_min);
 }
 
 /* tiles of the used slots of group g (g < 0: all groups) */
@@ -309,10 +327,54 @@ int eng_pick_rows(hype_engine *E)
     return best;
 }
 
+/* Heights for a mix of systems.  A Baer-Nunziato row takes three times as long as
+ * an Euler row, and the groups' launches run side by side, so one height for all
+ * leaves a stage waiting for a few tall Baer-Nunziato tiles while the rest of the
+ * device idles (16 grids of the three systems, 1.5 M cells: 40 rows, 4.5 ms a
+ * step).  The heights are instead in inverse proportion to a row's time, and the
+ * scale is the one with the least modelled time of a stage: the waves' total time
+ * over the device's SIMDs, plus the longest tile as the tail (1.7 ms a step). */
+int eng_auto_rows(hype_engine *E)
+{
+    const double simds = 4.0 * E->ncu;
+    double lo = 1e300, hi = 0.0, best_t = 1e300;
+    int s, h, best = 1;
+    for (s = 0; s < E->cap; ++s) {
+        double t;
+        if (!E->used[s] || !E->run[s]) continue;
+        t = tile_row_time(E, s);
+        if (t < lo) lo = t;
+        if (t > hi) hi = t;
+    }
+    if (hi <= 1.25 * lo) return eng_set_rows(E, eng_pick_rows(E));
+    for (h = 1; h <= 256; ++h) {
+        double work = 0.0, tail = 0.0;
+        for (s = 0; s < E->cap; ++s) {
+            const int bw = E->g[E->group_of[s]].bwaves;
+            int nsy;
+            double t;
+            if (!E->used[s] || !E->run[s]) continue;
+            nsy = rows_at(E, s, h, 1, lo);
+            t = hype_row_time(&E->P[s]) * hype_tile_rows((E->P[s].ny + nsy - 1) / nsy, bw > 1);
+            work += t * hype_strips(E->P[s].nx) * nsy * bw;
+            if (t > tail) tail = t;
+        }
+        if (work / simds + tail < best_t) {
+            best_t = work / simds + tail;
+            best = h;
+        }
+    }
+    E->target_rows = best;
+    E->weighted = 1;
+    E->row_min = lo;
+    return HYPE_OK;
+}
+
 int eng_set_rows(hype_engine *E, int rows)
 {
     if (rows < 1) return HYPE_E_INVALID;
     E->target_rows = rows;
+    E->weighted = 0;
     return HYPE_OK;
 }
 

@@ -50,7 +50,10 @@ typedef struct {
     hype_problem *P;
     int *used, *group_of, *nsy, *fresh;
     int *run;               /* used slots advanced by eng_step (default all) */
-    int target_rows;        /* common tile height of all instances */
+    int target_rows;        /* tile height of all instances, or (weighted) of
+                               those whose rows take the least time */
+    int weighted;           /* 1: heights in inverse proportion to a row's time */
+    double row_min;         /* least tile-row time of the running slots (weighted) */
     int layout;             /* tile layout where a system has both: -1 the
                                default (one wave per tile), 0 one wave, 1 split */
     eng_group g[HYPE_MAX_GROUPS];
@@ -93,8 +96,11 @@ int eng_start(hype_engine *E, const int *slots, int n, const double *t0, const d
 int eng_step(hype_engine *E, int nsteps);
 int eng_sync(hype_engine *E);
 int eng_read_states(hype_engine *E, hype_dstate *out);
-/* tile height the model picks for the used slots */
+/* common tile height the model picks for the running slots */
 int eng_pick_rows(hype_engine *E);
+/* set the tile heights the model picks for the running slots: common, or by
+ * system where their rows take different times */
+int eng_auto_rows(hype_engine *E);
 int eng_set_rows(hype_engine *E, int rows);
 int eng_total_tiles(hype_engine *E);
 

@@ -73,6 +73,7 @@ struct hype_server {
     long long active_cells;
     int *slot_req;          /* request resident in each slot, or -1 */
     long long *slot_round;  /* first round that steps the slot's request */
+    long long *slot_steps;  /* steps enqueued for the slot's request so far */
     int *order;             /* scratch for the running-set selection */
     double *key;
     int *fresh;             /* slots admitted in this poll */
@@ -202,6 +203,7 @@ void hype_server_destroy(hype_server *s)
     free(s->queue);
     free(s->slot_req);
     free(s->slot_round);
+    free(s->slot_steps);
     free(s->order);
     free(s->key);
     free(s->fresh);
@@ -253,6 +255,7 @@ int hype_server_create(const hype_server_opts *opts, hype_server **out)
     cap = s->o.max_active;
     s->slot_req = (int *)malloc((size_t)cap * sizeof(int));
     s->slot_round = (long long *)calloc((size_t)cap, sizeof(long long));
+    s->slot_steps = (long long *)calloc((size_t)cap, sizeof(long long));
     s->order = (int *)malloc((size_t)cap * sizeof(int));
     s->key = (double *)malloc((size_t)cap * sizeof(double));
     s->fresh = (int *)malloc((size_t)cap * sizeof(int));
@@ -261,7 +264,7 @@ int hype_server_create(const hype_server_opts *opts, hype_server **out)
     s->t_end = (double *)malloc((size_t)cap * sizeof(double));
     s->maxs = (int *)malloc((size_t)cap * sizeof(int));
     s->d = (hype_dstate *)calloc((size_t)cap, sizeof(hype_dstate));
-    if (!s->slot_req || !s->slot_round || !s->order || !s->key || !s->fresh || !s->clip || !s->t0 ||
+    if (!s->slot_req || !s->slot_round || !s->slot_steps || !s->order || !s->key || !s->fresh || !s->clip || !s->t0 ||
         !s->t_end || !s->maxs || !s->d) {
         hype_server_destroy(s);
         return HYPE_E_NOMEM;
@@ -362,6 +365,33 @@ static double remaining_work(const hype_server *s, int slot)
         }
     }
     return (double)q->r.problem.nx * q->r.problem.ny * hype_nvar(q->r.problem.system) * steps;
+}
+
+/* Steps worth enqueuing for the running instances: the most that any of them can
+ * still take after those already enqueued.  Its step budget is exact; where it
+ * ends by time, the steps to t_end at its last dt are an estimate, and an instance
+ * that turns out to need more gets them in later rounds.  Steps beyond this would
+ * run as launches that find every instance finished. */
+static int steps_left(const hype_server *s)
+{
+    long long most = 0;
+    int slot;
+    for (slot = 0; slot < s->o.max_active; ++slot) {
+        const srv_req *q;
+        long long left;
+        if (s->slot_req[slot] < 0 || !s->E.run[slot]) continue;
+        q = &s->req[s->slot_req[slot]];
+        left = q->r.max_steps - s->slot_steps[slot];
+        if (left > 0 && state_valid(s, slot)) {
+            const hype_dstate *d = &s->d[slot];
+            if (d->dt > 0.0 && d->t_end < 1e300) {
+                const double by_time = (d->t_end - d->t) / d->dt + 1.0 - (double)(s->slot_steps[slot] - d->step);
+                if (by_time < (double)left) left = by_time > 1.0 ? (long long)by_time : 1;
+            }
+        }
+        if (left > most) most = left;
+    }
+    return most < 256 ? (int)most : 256;
 }
 
 static int cmp_key(const void *a, const void *b, void *ctx)
@@ -512,6 +542,7 @@ int hype_server_poll(hype_server *s, int *active, int *queued)
         q->state = HYPE_REQ_RUNNING;
         q->t_start = t;
         s->slot_req[slot] = id;
+        s->slot_steps[slot] = 0;
         s->slot_round[slot] = s->round; /* primed and first stepped in the round enqueued below */
         s->fresh[nfresh] = slot;
         s->clip[nfresh] = (q->r.flags & HYPE_TS_CLIP) != 0;
@@ -532,7 +563,7 @@ int hype_server_poll(hype_server *s, int *active, int *queued)
      * copied behind the queued steps; the priming waits for the uploads */
     eng_flip(&s->E);
     if (changed) {
-        if (s->o.tile_rows < 1) eng_set_rows(&s->E, eng_pick_rows(&s->E));
+        if (s->o.tile_rows < 1) eng_auto_rows(&s->E);
         if ((rc = eng_commit(&s->E)) != HYPE_OK) goto out;
         if (nfresh > 0) {
             if ((rc = hyped_event_record(s->ev_up, s->copy)) != HYPE_OK) goto out;
@@ -550,6 +581,9 @@ int hype_server_poll(hype_server *s, int *active, int *queued)
             if (n < 1) n = 1;
             if (n > 256) n = 256;
         }
+        if (n > (k = steps_left(s))) n = k;
+        for (slot = 0; slot < s->o.max_active; ++slot)
+            if (s->slot_req[slot] >= 0 && s->E.run[slot]) s->slot_steps[slot] += n;
         if ((rc = hyped_event_record(s->ev0[p], s->E.stream)) != HYPE_OK) goto out;
         if ((rc = eng_step(&s->E, n)) != HYPE_OK) goto out;
         if ((rc = hyped_event_record(s->ev1[p], s->E.stream)) != HYPE_OK) goto out;
