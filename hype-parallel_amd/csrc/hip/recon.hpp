@@ -252,8 +252,17 @@ __device__ __forceinline__ bool weno3_fast(const double* U_x, const double* U_y,
 }
 
 // reconstruction.c:223-357: CWENO with one fourth-degree central candidate
-// and five third-degree candidates (gamma_hi = gamma_lo = 0.85)
-__device__ __forceinline__ void weno4(const double* U_x, const double* U_y, const double* U_xy, double* coeffs) {
+// and five third-degree candidates (gamma_hi = gamma_lo = 0.85).  FAST divides
+// with shared reciprocals, as weno3_fast does, and returns false where a divisor
+// is out of their range; the other form divides plainly.  The 13 divisions were
+// 182 of a component's issue slots and are 88; halving joins the additions where
+// the component is never subnormal (TINY as in weno3_dir).  Kapila 256x256, 3
+// RK104 steps: 1238 -> 1143 us; Baer-Nunziato 1024x1024, one step: 7642 -> 4319 us (its
+// registers no longer spill as far).
+template <bool FAST, bool TINY>
+__device__ __forceinline__ bool weno4(const double* U_x, const double* U_y, const double* U_xy, double* coeffs) {
+  // a + x / 2
+  auto add_half = [](double a, double x) { return TINY ? a + 0.5 * x : fma(0.5, x, a); };
   constexpr double r1_6 = 1. / 6., r13_3 = 13. / 3., r7_6 = 7. / 6., r11_120 = 11. / 120., r1_12 = 1. / 12.,
                    r41_60 = 41. / 60.;
   const double gammaHi = 0.85, gammaLo = 0.85;
@@ -270,60 +279,68 @@ __device__ __forceinline__ void weno4(const double* U_x, const double* U_y, cons
 
   const double xR4 = r41_60 * (-u_im1 + u_ip1) + r11_120 * (u_im2 - u_ip2);
   const double yR4 = r41_60 * (-u_jm1 + u_jp1) + r11_120 * (u_jm2 - u_jp2);
-  const double xxR4 = -u_0 + 0.5 * (u_im1 + u_ip1);
-  const double yyR4 = -u_0 + 0.5 * (u_jm1 + u_jp1);
+  const double xxR4 = add_half(-u_0, u_im1 + u_ip1);
+  const double yyR4 = add_half(-u_0, u_jm1 + u_jp1);
   const double xyR4 = 0.25 * (u_im1jm1 - u_im1jp1 - u_ip1jm1 + u_ip1jp1);
   const double xxxR4 = r1_6 * (u_im1 - u_ip1) + r1_12 * (u_ip2 - u_im2);
   const double yyyR4 = r1_6 * (u_jm1 - u_jp1) + r1_12 * (u_jp2 - u_jm2);
-  const double xxyR4 = 0.25 * (-u_im1jm1 + u_im1jp1 - u_ip1jm1 + u_ip1jp1) + 0.5 * (u_jm1 - u_jp1);
-  const double xyyR4 = 0.5 * (u_im1 - u_ip1) + 0.25 * (u_ip1jp1 - u_im1jm1 - u_im1jp1 + u_ip1jm1);
+  const double xxyR4 = add_half(0.25 * (-u_im1jm1 + u_im1jp1 - u_ip1jm1 + u_ip1jp1), u_jm1 - u_jp1);
+  const double xyyR4 = add_half(0.25 * (u_ip1jp1 - u_im1jm1 - u_im1jp1 + u_ip1jm1), u_im1 - u_ip1);
   const double IS_R4 = (xR4 + 0.1 * xxxR4) * (xR4 + 0.1 * xxxR4) + r13_3 * (xxR4 * xxR4 + yyR4 * yyR4) +
                        (yR4 + 0.1 * yyyR4) * (yR4 + 0.1 * yyyR4) + 39.05 * (xxxR4 * xxxR4 + yyyR4 * yyyR4) +
                        r7_6 * xyR4 * xyR4 + 4.7 * (xxyR4 * xxyR4 + xyyR4 * xyyR4);
-  double wR4 = gR4 / (pow4(IS_R4 + SMALL_NUM));
+  unsigned top = 0;
+  auto weight = [&](double g, double IS) {
+    const double d = pow4(IS + SMALL_NUM);
+    top = max(top, hi_word(d));
+    return FAST ? div_y(g, d, recip_nr(d)) : g / d;
+  };
+  double wR4 = weight(gR4, IS_R4);
   double sum = wR4;
 
   xR3[0] = 0.5 * (-u_im1 + u_ip1);
   yR3[0] = 0.5 * (-u_jm1 + u_jp1);
-  xxR3[0] = -u_0 + 0.5 * (u_im1 + u_ip1);
-  yyR3[0] = -u_0 + 0.5 * (u_jm1 + u_jp1);
-  xyR3[0] = 0.25 * (u_im1jm1 - u_im1jp1 - u_ip1jm1 + u_ip1jp1);
+  xxR3[0] = xxR4;
+  yyR3[0] = yyR4;
+  xyR3[0] = xyR4;
 
-  xR3[1] = 1.5 * u_0 - 2.0 * u_im1 + 0.5 * u_im2;
+  xR3[1] = add_half(fma(-2.0, u_im1, 1.5 * u_0), u_im2);
   yR3[1] = 0.5 * (-u_jm1 + u_jp1);
-  xxR3[1] = 0.5 * u_0 - u_im1 + 0.5 * u_im2;
-  yyR3[1] = -u_0 + 0.5 * u_jm1 + 0.5 * u_jp1;
+  xxR3[1] = add_half(add_half(-u_im1, u_0), u_im2);
+  yyR3[1] = add_half(add_half(-u_0, u_jm1), u_jp1);
   xyR3[1] = 0.5 * (u_im1jm1 - u_im1jp1 - u_jm1 + u_jp1);
 
-  xR3[2] = -1.5 * u_0 + 2.0 * u_ip1 - 0.5 * u_ip2;
+  xR3[2] = add_half(fma(2.0, u_ip1, -1.5 * u_0), -u_ip2);
   yR3[2] = 0.5 * (-u_jm1 + u_jp1);
-  xxR3[2] = 0.5 * u_0 - u_ip1 + 0.5 * u_ip2;
-  yyR3[2] = -u_0 + 0.5 * u_jm1 + 0.5 * u_jp1;
+  xxR3[2] = add_half(add_half(-u_ip1, u_0), u_ip2);
+  yyR3[2] = yyR3[1];
   xyR3[2] = 0.5 * (-u_ip1jm1 + u_ip1jp1 + u_jm1 - u_jp1);
 
   xR3[3] = 0.5 * (-u_im1 + u_ip1);
-  yR3[3] = 1.5 * u_0 - 2.0 * u_jm1 + 0.5 * u_jm2;
-  xxR3[3] = -u_0 + 0.5 * u_im1 + 0.5 * u_ip1;
-  yyR3[3] = 0.5 * u_0 - u_jm1 + 0.5 * u_jm2;
+  yR3[3] = add_half(fma(-2.0, u_jm1, 1.5 * u_0), u_jm2);
+  xxR3[3] = add_half(add_half(-u_0, u_im1), u_ip1);
+  yyR3[3] = add_half(add_half(-u_jm1, u_0), u_jm2);
   xyR3[3] = 0.5 * (-u_im1 + u_im1jm1 + u_ip1 - u_ip1jm1);
 
   xR3[4] = 0.5 * (-u_im1 + u_ip1);
-  yR3[4] = -1.5 * u_0 + 2.0 * u_jp1 - 0.5 * u_jp2;
-  xxR3[4] = -u_0 + 0.5 * u_im1 + 0.5 * u_ip1;
-  yyR3[4] = 0.5 * u_0 - u_jp1 + 0.5 * u_jp2;
+  yR3[4] = add_half(fma(2.0, u_jp1, -1.5 * u_0), -u_jp2);
+  xxR3[4] = xxR3[3];
+  yyR3[4] = add_half(add_half(-u_jp1, u_0), u_jp2);
   xyR3[4] = 0.5 * (u_im1 - u_im1jp1 - u_ip1 + u_ip1jp1);
 
 #pragma unroll
   for (int i = 0; i < 5; ++i) {
     const double IS = xR3[i] * xR3[i] + yR3[i] * yR3[i] + r13_3 * (xxR3[i] * xxR3[i] + yyR3[i] * yyR3[i]) +
                       r7_6 * xyR3[i] * xyR3[i];
-    wR3[i] = gR3[i] / (pow4(IS + SMALL_NUM));
+    wR3[i] = weight(gR3[i], IS);
     sum = sum + wR3[i];
   }
-  wR4 = wR4 / sum;
+  const double ys = recip_nr(sum);
+  wR4 = FAST ? div_y(wR4, sum, ys) : wR4 / sum;
 #pragma unroll
-  for (int i = 0; i < 5; ++i) wR3[i] = wR3[i] / sum;
-  const double wt_ratio = wR4 / gR4;
+  for (int i = 0; i < 5; ++i) wR3[i] = FAST ? div_y(wR3[i], sum, ys) : wR3[i] / sum;
+  constexpr double yg = 1.0 / 0.85;  // rounded, as div_y needs it
+  const double wt_ratio = FAST ? div_y(wR4, gR4, yg) : wR4 / gR4;
 
   auto coef = [&](double R4, const double* R3) {
     return wt_ratio * (R4 - gR3[0] * R3[0] - gR3[1] * R3[1] - gR3[2] * R3[2] - gR3[3] * R3[3] - gR3[4] * R3[4]) +
@@ -339,6 +356,7 @@ __device__ __forceinline__ void weno4(const double* U_x, const double* U_y, cons
   coeffs[7] = wt_ratio * yyyR4;
   coeffs[8] = wt_ratio * xxyR4;
   coeffs[9] = wt_ratio * xyyR4;
+  return top < FDIV_TOP_WORD;
 }
 
 // Stencil of one component: x[0..4] = u(i-2..i+2, j), y[0..4] = u(i, j-2..j+2),
@@ -356,7 +374,7 @@ __device__ __forceinline__ void reconstruct(const double* U_x, const double* U_y
     coeffs[1] = minmod(U_x[3] - u_0, u_0 - U_x[1]);
     coeffs[2] = minmod(U_y[3] - u_0, u_0 - U_y[1]);
   } else if constexpr (N == 3) {
-    weno4(U_x, U_y, U_xy, coeffs);
+    if (!__builtin_expect((weno4<true, TINY>(U_x, U_y, U_xy, coeffs)), 1)) weno4<false, TINY>(U_x, U_y, U_xy, coeffs);
   } else {
     if (__builtin_expect(weno3_fast<TINY>(U_x, U_y, U_xy, coeffs), 1)) return;
     // reconstruction.c:144-221
