@@ -118,25 +118,30 @@ struct Duo {
     auto P_ = [&](int k) -> double& { return part[k * HYPE_WAVE + lane]; };
 
     // ---- row loader (as in Tile) ---------------------------------------
-    auto fetch = [&](int rr, int k, double* q) -> int {
-      const int cc = min(x0 - 3 + k, nx + 2);
-      bool fx = false, fy = false;
-      const int sc = bc_map(cc, nx, bcL, bcR, fx);
+    // a cell's column is the same in every row: its source offset and the sign its
+    // reflection gives the x velocity are found once (lane k's window column, and
+    // the one right of the lanes' 64 that lanes 0-3, or all in turn, load)
+    auto column = [&](int k, unsigned& mx) -> size_t {
+      bool fx = false;
+      const int sc = bc_map(min(x0 - 3 + k, nx + 2), nx, bcL, bcR, fx);  // an inlet column maps as periodic; put_inlet replaces it
+      mx = fx ? SIGN_BIT : 0u;
+      return (size_t)sc * NV;
+    };
+    unsigned mxa, mxb;
+    const size_t cola = column(lane, mxa), colb = column(HYPE_WAVE + (lane & 3), mxb);
+    auto fetch = [&](int rr, size_t co, double* q) -> unsigned {
+      bool fy = false;
       const int sr = bc_map(rr, ny, bcB, bcT, fy);
-      const auto p = Uin + ((size_t)sr * nx + sc) * NV;
+      const auto p = Uin + (size_t)sr * nx * NV + co;
 #pragma unroll
       for (int c = 0; c < NV; ++c) q[c] = p[c];
-      return (fx ? 1 : 0) | (fy ? 2 : 0);
+      return fy ? SIGN_BIT : 0u;
     };
-    auto conv = [&](double* q, int refl, double* v) {
-      if (refl & 1) {
-        q[S::REFX[0]] = -q[S::REFX[0]];
-        if (S::REFX[1] >= 0) q[S::REFX[1]] = -q[S::REFX[1]];
-      }
-      if (refl & 2) {
-        q[S::REFY[0]] = -q[S::REFY[0]];
-        if (S::REFY[1] >= 0) q[S::REFY[1]] = -q[S::REFY[1]];
-      }
+    auto conv = [&](double* q, unsigned mx, unsigned my, double* v) {
+      q[S::REFX[0]] = flip_sign(q[S::REFX[0]], mx);
+      if (S::REFX[1] >= 0) q[S::REFX[1]] = flip_sign(q[S::REFX[1]], mx);
+      q[S::REFY[0]] = flip_sign(q[S::REFY[0]], my);
+      if (S::REFY[1] >= 0) q[S::REFY[1]] = flip_sign(q[S::REFY[1]], my);
       if (PRIM) {
         S::cons2prim(eos, q, v);
       } else {
@@ -144,9 +149,9 @@ struct Duo {
         for (int c = 0; c < NV; ++c) v[c] = q[c];
       }
     };
-    auto put = [&](int s, int k, double* q, int refl) {
+    auto put = [&](int s, int k, double* q, unsigned mx, unsigned my) {
       double v[NV];
-      conv(q, refl, v);
+      conv(q, mx, my, v);
 #pragma unroll
       for (int c = 0; c < NV; ++c) W_(s, c, k) = v[c];
     };
@@ -154,9 +159,9 @@ struct Duo {
     // converted 16 rows at a time, one cell per lane, and copied a row at a time
     // by lanes 0-3; on the conservative path loaded by lanes 0-3 with each row
     auto xrow = [&](int j0) { return rbase + j0 + (lane >> 2); };
-    auto xput = [&](double* q, int refl) {
+    auto xput = [&](double* q, unsigned my) {
       double v[NV];
-      conv(q, refl, v);
+      conv(q, mxb, my, v);
 #pragma unroll
       for (int c = 0; c < NV; ++c) xs[c * HYPE_WAVE + lane] = v[c];
     };
@@ -190,13 +195,13 @@ struct Duo {
     // prologue: rows r_first-2 .. r_first+2, three by wave X and two with the
     // right-hand columns by wave Y, in flight before the time state is read
     double pq[3][NV], pqb[NV];
-    int pf[3] = {0, 0, 0}, pfb = 0;
+    unsigned pf[3] = {0, 0, 0}, pfb = 0;
     const int pr0 = wave == 0 ? 0 : 3, prn = wave == 0 ? 3 : 2;
     const bool pxl = wave == 1 && (PRIM ? xrow(0) <= r_last + 2 : lane < 20);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
-      if (i < prn) pf[i] = fetch(rbase + pr0 + i, lane, pq[i]);
-    if (pxl) pfb = fetch(xrow(0), HYPE_WAVE + (lane & 3), pqb);
+      if (i < prn) pf[i] = fetch(rbase + pr0 + i, cola, pq[i]);
+    if (pxl) pfb = fetch(xrow(0), colb, pqb);
 
     // ---- time state (single writer per field per launch; as in Tile) -----
     if (mode == HYPE_MODE_STAGE) {
@@ -233,7 +238,7 @@ struct Duo {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
       if (i < prn) {
-        put(slot(rbase + pr0 + i), lane, pq[i], pf[i]);
+        put(slot(rbase + pr0 + i), lane, pq[i], mxa, pf[i]);
         put_inlet(slot(rbase + pr0 + i), rbase + pr0 + i);
       }
     if (wave == 1) {
@@ -243,7 +248,7 @@ struct Duo {
 #pragma unroll
         for (int i = 0; i < 5; ++i) xcopy(slot(rbase + i), i);
       } else {
-        if (pxl) put(slot(rbase + (lane >> 2)), HYPE_WAVE + (lane & 3), pqb, pfb);
+        if (pxl) put(slot(rbase + (lane >> 2)), HYPE_WAVE + (lane & 3), pqb, mxb, pfb);
       }
     }
     __syncthreads();
@@ -399,14 +404,14 @@ struct Duo {
         const bool xb = PRIM && more && (jn & 15) == 0;
         const bool xl = xb && xrow(jn) <= r_last + 2;
         double qa[NV], qb[NV];
-        int fa = 0, fb = 0;
+        unsigned fa = 0, fb = 0;
         if constexpr (!X) {
           if (more) {
-            fa = fetch(r + 3, lane, qa);
+            fa = fetch(r + 3, cola, qa);
             if constexpr (PRIM) {
-              if (xl) fb = fetch(xrow(jn), HYPE_WAVE + (lane & 3), qb);
+              if (xl) fb = fetch(xrow(jn), colb, qb);
             } else {
-              if (lane < 4) fb = fetch(r + 3, lane + HYPE_WAVE, qb);
+              if (lane < 4) fb = fetch(r + 3, colb, qb);
             }
           }
         }
@@ -454,7 +459,7 @@ struct Duo {
           }
         } else if (more) {  // row r+3 takes the slot of row r-2
           const int sn = slot(r + 3);
-          put(sn, lane, qa, fa);
+          put(sn, lane, qa, mxa, fa);
           if constexpr (PRIM) {
             if (xb) {
               if (xl) xput(qb, fb);
@@ -462,7 +467,7 @@ struct Duo {
             }
             xcopy(sn, jn);
           } else {
-            if (lane < 4) put(sn, lane + HYPE_WAVE, qb, fb);
+            if (lane < 4) put(sn, lane + HYPE_WAVE, qb, mxb, fb);
           }
           put_inlet(sn, r + 3);
         }

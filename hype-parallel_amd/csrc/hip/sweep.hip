@@ -130,6 +130,12 @@ __device__ __forceinline__ int bc_map(int i, int n, int bclo, int bchi, bool& fl
   return i;
 }
 
+// negates v where m is the sign bit, leaves it where m is 0
+__device__ __forceinline__ double flip_sign(double v, unsigned m) {
+  return __hiloint2double(__double2hiint(v) ^ (int)m, __double2loint(v));
+}
+constexpr unsigned SIGN_BIT = 0x80000000u;
+
 __device__ __forceinline__ double wave_max(double v) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
@@ -409,27 +415,32 @@ struct Tile {
 
     // ---- row loader ----------------------------------------------------
     // fetch issues the loads of one cell (source cell from the boundary
-    // index maps) and returns its reflection flags; put applies them, so a
+    // index maps) and returns its row's reflection; put applies it, so a
     // row's loads need not complete before the next row's are issued
-    auto fetch = [&](int rr, int k, double* q) -> int {
-      const int cc = min(x0 - 3 + k, nx + 2);
-      bool fx = false, fy = false;
-      const int sc = bc_map(cc, nx, bcL, bcR, fx);  // an inlet column maps as periodic; put_inlet replaces it
+    // a cell's column is the same in every row: its source offset and the sign its
+    // reflection gives the x velocity are found once (lane k's window column, and
+    // the one right of the lanes' 64 that lanes 0-3, or all in turn, load)
+    auto column = [&](int k, unsigned& mx) -> size_t {
+      bool fx = false;
+      const int sc = bc_map(min(x0 - 3 + k, nx + 2), nx, bcL, bcR, fx);  // an inlet column maps as periodic; put_inlet replaces it
+      mx = fx ? SIGN_BIT : 0u;
+      return (size_t)sc * NV;
+    };
+    unsigned mxa, mxb;
+    const size_t cola = column(lane, mxa), colb = column(HYPE_WAVE + (lane & 3), mxb);
+    auto fetch = [&](int rr, size_t co, double* q) -> unsigned {
+      bool fy = false;
       const int sr = bc_map(rr, ny, bcB, bcT, fy);
-      const auto p = Uin + ((size_t)sr * nx + sc) * NV;
+      const auto p = Uin + (size_t)sr * nx * NV + co;
 #pragma unroll
       for (int c = 0; c < NV; ++c) q[c] = p[c];
-      return (fx ? 1 : 0) | (fy ? 2 : 0);
+      return fy ? SIGN_BIT : 0u;
     };
-    auto conv = [&](double* q, int refl, double* v) {
-      if (refl & 1) {
-        q[S::REFX[0]] = -q[S::REFX[0]];
-        if (S::REFX[1] >= 0) q[S::REFX[1]] = -q[S::REFX[1]];
-      }
-      if (refl & 2) {
-        q[S::REFY[0]] = -q[S::REFY[0]];
-        if (S::REFY[1] >= 0) q[S::REFY[1]] = -q[S::REFY[1]];
-      }
+    auto conv = [&](double* q, unsigned mx, unsigned my, double* v) {
+      q[S::REFX[0]] = flip_sign(q[S::REFX[0]], mx);
+      if (S::REFX[1] >= 0) q[S::REFX[1]] = flip_sign(q[S::REFX[1]], mx);
+      q[S::REFY[0]] = flip_sign(q[S::REFY[0]], my);
+      if (S::REFY[1] >= 0) q[S::REFY[1]] = flip_sign(q[S::REFY[1]], my);
       if (PRIM) {
         S::cons2prim(eos, q, v);
       } else {
@@ -437,9 +448,9 @@ struct Tile {
         for (int c = 0; c < NV; ++c) v[c] = q[c];
       }
     };
-    auto put = [&](int s, int k, double* q, int refl) {
+    auto put = [&](int s, int k, double* q, unsigned mx, unsigned my) {
       double v[NV];
-      conv(q, refl, v);
+      conv(q, mx, my, v);
 #pragma unroll
       for (int c = 0; c < NV; ++c) W_(s, c, k) = v[c];
     };
@@ -453,9 +464,9 @@ struct Tile {
     // needed and not loaded
     double* xs = wave == 0 ? xch : lds + WAVES * WIN + (PAIR ? 2 * XCH + DEFER : 0) + WAVES * OST + (COMBINE ? 1 : 0);
     auto xrow = [&](int j0) { return rbase + j0 + (lane >> 2); };
-    auto xput = [&](double* q, int refl) {
+    auto xput = [&](double* q, unsigned my) {
       double v[NV];
-      conv(q, refl, v);
+      conv(q, mxb, my, v);
 #pragma unroll
       for (int c = 0; c < NV; ++c) xs[c * HYPE_WAVE + lane] = v[c];
     };
@@ -495,19 +506,19 @@ struct Tile {
     // first store, and before the time state is read: it decides whether the
     // tile runs at all, and its round trip now overlaps theirs
     double pqa[5][NV], pqb[5][NV];
-    int pfa[5], pfb[5];
+    unsigned pfa[5], pfb[5];
     const bool pxl = XBATCH && xrow(0) <= r_last + 2;
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
-      pfa[i] = fetch(rbase + i, lane, pqa[i]);
+      pfa[i] = fetch(rbase + i, cola, pqa[i]);
       pfb[i] = 0;
     }
     if constexpr (XBATCH) {
-      if (pxl) pfb[0] = fetch(xrow(0), HYPE_WAVE + (lane & 3), pqb[0]);
+      if (pxl) pfb[0] = fetch(xrow(0), colb, pqb[0]);
     } else {
 #pragma unroll
       for (int i = 0; i < 5; ++i)
-        if (lane < 4) pfb[i] = fetch(rbase + i, lane + HYPE_WAVE, pqb[i]);
+        if (lane < 4) pfb[i] = fetch(rbase + i, colb, pqb[i]);
     }
 
     // ---- time state (single writer per field per launch) -------------
@@ -547,7 +558,7 @@ struct Tile {
     if constexpr (XBATCH) {
 #pragma unroll
       for (int i = 0; i < 5; ++i) {
-        put(slot(rbase + i), lane, pqa[i], pfa[i]);
+        put(slot(rbase + i), lane, pqa[i], mxa, pfa[i]);
         put_inlet(slot(rbase + i), rbase + i);
       }
       if (pxl) xput(pqb[0], pfb[0]);
@@ -557,8 +568,8 @@ struct Tile {
     } else {
 #pragma unroll
       for (int i = 0; i < 5; ++i) {
-        put(slot(rbase + i), lane, pqa[i], pfa[i]);
-        if (lane < 4) put(slot(rbase + i), lane + HYPE_WAVE, pqb[i], pfb[i]);
+        put(slot(rbase + i), lane, pqa[i], mxa, pfa[i]);
+        if (lane < 4) put(slot(rbase + i), lane + HYPE_WAVE, pqb[i], mxb, pfb[i]);
         put_inlet(slot(rbase + i), rbase + i);
       }
     }
@@ -730,13 +741,13 @@ struct Tile {
       const bool xb = XBATCH && more && (jn & 15) == 0;
       const bool xl = xb && xrow(jn) <= r_last + 2;
       double qa[NV], qb[NV];
-      int fa = 0, fb = 0;
+      unsigned fa = 0, fb = 0;
       if (more) {
-        fa = fetch(r + 3, lane, qa);
+        fa = fetch(r + 3, cola, qa);
         if constexpr (XBATCH) {
-          if (xl) fb = fetch(xrow(jn), HYPE_WAVE + (lane & 3), qb);
+          if (xl) fb = fetch(xrow(jn), colb, qb);
         } else {
-          if (lane < 4) fb = fetch(r + 3, lane + HYPE_WAVE, qb);
+          if (lane < 4) fb = fetch(r + 3, colb, qb);
         }
       }
 
@@ -805,7 +816,7 @@ struct Tile {
       // slot (the wave's own reads above precede this store in program order)
       if (more) {
         const int sn = slot(r + 3);
-        put(sn, lane, qa, fa);
+        put(sn, lane, qa, mxa, fa);
         if constexpr (XBATCH) {
           if (xb) {
             if (xl) xput(qb, fb);
@@ -813,7 +824,7 @@ struct Tile {
           }
           xcopy(sn, jn);
         } else {
-          if (lane < 4) put(sn, lane + HYPE_WAVE, qb, fb);
+          if (lane < 4) put(sn, lane + HYPE_WAVE, qb, mxb, fb);
         }
         put_inlet(sn, r + 3);
       }
