@@ -236,6 +236,14 @@ struct Tile {
   static constexpr int WAVES = PAIR ? 2 : 1;
   // the admissibility check's a_sq at each node goes on to the flux there
   static constexpr bool ACACHE = PRIM && S::HAS_ACACHE && N == 2;
+  // conservative path, one wave per tile, few nodes (4 at orders 0 and 1; at order
+  // 2 the 8 nodes' fluxes do not fit): the flux and wave speed of a node's state
+  // are computed where its admissibility is checked and go to the face with it,
+  // so the two share a division and the pressure.  Euler minmod 1535x1023: 110.1
+  // -> 106.2 us per step, Baer-Nunziato order 1 1024x512 156.9 -> 147.7.  Not for
+  // split tiles, whose ring rows need no flux (Euler 256x256: 28.3 -> 28.5), nor
+  // Kapila, whose flux shares too little with its check (1024x512: 105.7 -> 112.2)
+  static constexpr bool SIDES = !PRIM && N <= 1 && !PAIR;
   // inadmissible states are looked for after each face point where the states
   // of a face's points are too many to be kept (nine components: 191 registers
   // spilled), else once per face, which leaves its arithmetic in one block
@@ -281,6 +289,38 @@ struct Tile {
   // reference's operations
   static constexpr bool plain(int dir, int c) {
     return S::JUMP_TINY[c] || c == (dir == 0 ? S::REFY : S::REFX)[0] || c == (dir == 0 ? S::REFY : S::REFX)[1];
+  }
+  // flux and wave speed of a conserved state (SIDES)
+  struct Side {
+    double F[SIDES ? NV : 1], s;
+    bool bad;
+    template <int dir>
+    __device__ __forceinline__ void of(const Eos& e, const double* Q) {
+      bad = false;
+      s = S::template side_cons<dir>(e, Q, F, bad);
+    }
+    __device__ __forceinline__ Side from_left() const {
+      Side o;
+#pragma unroll
+      for (int c = 0; c < NV; ++c) o.F[c] = S::FZERO[c] ? 0.0 : lane_from_left(F[c]);
+      o.s = lane_from_left(s);
+      o.bad = lane_from_left_int(bad) != 0;
+      return o;
+    }
+  };
+  // riemann() from the sides
+  template <int dir>
+  __device__ static __forceinline__ double join(const Eos& e, const double* Lv, const double* Rv, const Side& Ls,
+                                                const Side& Rs, double* A, double* D, bool& bad) {
+    const double s = pmax(Ls.s, Rs.s);
+    bad = Ls.bad | Rs.bad;
+#pragma unroll
+    for (int c = 0; c < NV; ++c) {
+      const double dQ = Rv[c] - Lv[c];
+      A[c] = S::FZERO[c] ? -(s * dQ) : Rs.F[c] + Ls.F[c] - s * dQ;
+    }
+    S::template ncp_face<PRIM, dir>(e, Lv, Rv, D);
+    return s;
   }
   // add point q's flux A and jump D to the sums F and E of a face
   template <int dir>
@@ -578,6 +618,7 @@ struct Tile {
     // ---- carried state -------------------------------------------------
     double topPrev[NGF][NV];
     double topA[NGF];  // a_sq handed over with topPrev
+    Side topS[SIDES ? NGF : 1] = {};  // its sides
     // the face sums G, E (and Fx, Dx) of most components are kept unscaled (PLAIN
     // says which are not)
     double Gprev[NV], Eprev[NV], xpartPrev[NV], ncpPrev[NV];
@@ -609,12 +650,15 @@ struct Tile {
     // flux + jump sums at the y-face below row fr from the values either side
     // (lower side: top values of row fr-1; upper side: bottom values of fr)
     auto yface = [&](const double (&Lv)[NGF][NV], const double (&Rv)[NGF][NV], const double* aL, const double* aR,
-                     int fr, double* G, double* E) {
+                     const Side* sL, const Side* sR, int fr, double* G, double* E) {
       bool bad[NGF], any = false;
 #pragma unroll
       for (int q = 0; q < NGF; ++q) {
-        double A[NV], D[NV];
-        const double sp = riemann<S, PRIM, ACACHE, 1>(eos, Lv[q], Rv[q], A, D, bad[q], aL[q], aR[q]);
+        double A[NV], D[NV], sp;
+        if constexpr (SIDES)
+          sp = join<1>(eos, Lv[q], Rv[q], sL[q], sR[q], A, D, bad[q]);
+        else
+          sp = riemann<S, PRIM, ACACHE, 1>(eos, Lv[q], Rv[q], A, D, bad[q], aL[q], aR[q]);
         smax_y = fmax(smax_y, sp);
         any |= bad[q];
         if constexpr (CHECK_EACH) {
@@ -785,14 +829,32 @@ struct Tile {
       // ACACHE the check's a_sq at each node goes on to the flux there
       double an[ACACHE ? NNODE : 1];
       bool pad = true;
+      Side sd[SIDES ? NNODE : 1];
+      auto sides = [&]() {
+        if constexpr (SIDES) {
+#pragma unroll
+          for (int q = 0; q < NGF; ++q) {
+            sd[Qd::R(q)].template of<0>(eos, fv[Qd::R(q)]);
+            sd[Qd::L(q)].template of<0>(eos, fv[Qd::L(q)]);
+            sd[Qd::T(q)].template of<1>(eos, fv[Qd::T(q)]);
+            sd[Qd::B(q)].template of<1>(eos, fv[Qd::B(q)]);
+          }
+        }
+      };
+      sides();
 #pragma unroll
       for (int p = 0; p < NNODE; ++p) {
         if constexpr (ACACHE)
           pad = S::pad_prim_a(eos, fv[p], an[p]) && pad;
+        else if constexpr (SIDES)
+          pad = S::pad(eos, fv[p]) & pad;  // no branches: the flux computes it all
         else
           pad = pad && (PRIM ? S::pad_prim(eos, fv[p]) : S::pad(eos, fv[p]));
       }
-      if (!pad) {  // rhs_function_prim.c:407-421 / rhs_function.c:409-421
+      // rhs_function_prim.c:407-421 / rhs_function.c:409-421.  With SIDES the rare
+      // branch is the wave's: the compiler turned the lanes' into selects, and the
+      // flux of the cell's value into work of every row
+      if ((!SIDES || __builtin_expect(__ballot(!pad) != 0, 0)) && !pad) {
 #pragma unroll
         for (int c = 0; c < NV; ++c) {
           const double w0 = W_(s0, c, cw);
@@ -809,6 +871,7 @@ struct Tile {
 #pragma unroll
           for (int p = 0; p < NNODE; ++p) an[p] = S::sound_sq_prim(eos, fv[p]);
         }
+        sides();
       }
       if (L.fallback && ownedRow && owned) gmem(L.fallback)[(size_t)r * nx + col] = (unsigned char)(!pad);
 
@@ -857,10 +920,12 @@ struct Tile {
           Dx[c] = 0.0;
         }
         double vl[NGF][NV];
+        Side sl[SIDES ? NGF : 1];
 #pragma unroll
         for (int q = 0; q < NGF; ++q) {
 #pragma unroll
           for (int c = 0; c < NV; ++c) vl[q][c] = lane_from_left(fv[Qd::R(q)][c]);
+          if constexpr (SIDES) sl[q] = sd[Qd::R(q)].from_left();
           bad[q] = false;
           double al = 0.0, ar = 0.0;
           if constexpr (ACACHE) {
@@ -868,8 +933,11 @@ struct Tile {
             ar = an[Qd::L(q)];
           }
           if (ownedRow) {
-            double A[NV], D[NV];
-            const double s = riemann<S, PRIM, ACACHE, 0>(eos, vl[q], fv[Qd::L(q)], A, D, bad[q], al, ar);
+            double A[NV], D[NV], s;
+            if constexpr (SIDES)
+              s = join<0>(eos, vl[q], fv[Qd::L(q)], sl[q], sd[Qd::L(q)], A, D, bad[q]);
+            else
+              s = riemann<S, PRIM, ACACHE, 0>(eos, vl[q], fv[Qd::L(q)], A, D, bad[q], al, ar);
             smax_x = fmax(smax_x, s);
             any |= bad[q];
             if constexpr (CHECK_EACH) {
@@ -901,7 +969,12 @@ struct Tile {
         for (int q = 0; q < NGF; ++q)
 #pragma unroll
           for (int c = 0; c < NV; ++c) fvb[q][c] = fv[Qd::B(q)][c];
-        yface(topPrev, fvb, topA, an_b, r, Gy, Ey);
+        Side sb[SIDES ? NGF : 1];
+        if constexpr (SIDES) {
+#pragma unroll
+          for (int q = 0; q < NGF; ++q) sb[q] = sd[Qd::B(q)];
+        }
+        yface(topPrev, fvb, topA, an_b, topS, sb, r, Gy, Ey);
       } else {
 #pragma unroll
         for (int c = 0; c < NV; ++c) {
@@ -945,6 +1018,10 @@ struct Tile {
       if constexpr (ACACHE) {
 #pragma unroll
         for (int q = 0; q < NGF; ++q) topA[q] = an[Qd::T(q)];
+      }
+      if constexpr (SIDES) {
+#pragma unroll
+        for (int q = 0; q < NGF; ++q) topS[q] = sd[Qd::T(q)];
       }
 
       sync_window();  // the new row is visible to the next iteration
@@ -992,7 +1069,15 @@ struct Tile {
           ahi[q] = X_(1, q, NV);
         }
         double Gm[NV], Em[NV];
-        yface(lo, hi, alo, ahi, ym, Gm, Em);
+        Side slo[SIDES ? NGF : 1], shi[SIDES ? NGF : 1];
+        if constexpr (SIDES) {
+#pragma unroll
+          for (int q = 0; q < NGF; ++q) {
+            slo[q].template of<1>(eos, lo[q]);
+            shi[q].template of<1>(eos, hi[q]);
+          }
+        }
+        yface(lo, hi, alo, ahi, slo, shi, ym, Gm, Em);
         if (!upper) {
           assemble(ym - 1, Gm, Gprev, Em, Eprev, xpartPrev, ncpPrev, false);
         } else {
