@@ -244,6 +244,12 @@ struct Tile {
   // split tiles, whose ring rows need no flux (Euler 256x256: 28.3 -> 28.5), nor
   // Kapila, whose flux shares too little with its check (1024x512: 105.7 -> 112.2)
   static constexpr bool SIDES = !PRIM && N <= 1 && !PAIR;
+  // the stage update's operands are loaded half a row ahead of their use, which
+  // hides their round trip: Euler minmod 1535x1023 106.1 -> 101.2 us per step,
+  // Euler order 2 1024x1024 388 -> 382, Kapila 2048x1024 1316 -> 1307.  Not at order
+  // 3, whose registers are full (Euler 1024x1024: 1237 -> 1265, Baer-Nunziato: 2411
+  // -> 2521)
+  static constexpr bool AHEAD = N <= 2;
   // inadmissible states are looked for after each face point where the states
   // of a face's points are too many to be kept (nine components: 191 registers
   // spilled), else once per face, which leaves its arithmetic in one block
@@ -694,22 +700,46 @@ struct Tile {
       wave_sync();  // the staging is rewritten by the next row
     };
 
-    // an operand of the stage update read from buffer B.  On the
-    // conservative path the window holds the stage input of the owned cells
-    // unchanged, so while the row is still in the window (wr) the input is
-    // taken from there instead of being read from memory a second time
-    auto operand = [&](gmem_t<const double>* B, size_t i, int row, int c, bool wr) -> double {
-      if constexpr (!PRIM) {
+    // the operands of the stage update of cell (col, row): o0 is the AXPY's vector
+    // or X, o1 is Z or RK104's U.  Every operand of a record is loaded before its
+    // first store: the compiler cannot prove the output distinct from the inputs
+    // (it is not, for the RK stages that update U in place), so loads among the
+    // stores would each wait for memory.  With AHEAD they are loaded in the middle
+    // of the row's iteration and used at its end.  On the conservative path the window holds the stage input of the
+    // owned cells unchanged, so while the row is in the window (wr) that operand is
+    // taken from there (from) and not loaded
+    const auto B0 = mode == HYPE_MODE_STAGE && sd.op == 1 ? Xb : Uin;
+    const auto B1 = sd.op == 2 ? gmem<const double>(I->buf[sd.out]) : Zb;
+    auto operands = [&](int row, double (&o0)[NV], double (&o1)[NV], bool wr) {
+      if (mode != HYPE_MODE_STAGE || !owned) return;
+      const size_t idx = ((size_t)row * nx + col) * NV;
+      if (PRIM || !wr || B0 != Uin) {
+#pragma unroll
+        for (int c = 0; c < NV; ++c) o0[c] = B0[idx + c];
+      }
+      if (sd.op != 0 && (PRIM || !wr || B1 != Uin)) {
+#pragma unroll
+        for (int c = 0; c < NV; ++c) o1[c] = B1[idx + c];
+      }
+    };
+    auto from = [&](double o, gmem_t<const double>* B, int row, int c, bool wr) -> double {
+      if constexpr (!PRIM && AHEAD) {
         if (wr && B == Uin) return W_(slot(row), c, lane + 2);
       }
-      return B[i];
+      return o;
+    };
+    auto load = [&](double (&o)[NV], gmem_t<const double>* B, size_t idx, int row, bool wr) {  // without AHEAD
+      if constexpr (!AHEAD) {
+#pragma unroll
+        for (int c = 0; c < NV; ++c) o[c] = !PRIM && wr && B == Uin ? W_(slot(row), c, lane + 2) : B[idx + c];
+      }
     };
 
     // assembly + stage update of cell (col, row) from the terms of its top
     // and bottom faces, its x-face part and its volume term
     // (rhs_function_prim.c:589-602)
     auto record = [&](int row, const double* Gt, const double* Gb, const double* Et, const double* Eb,
-                      const double* xp, const double* nc, bool wr) {
+                      const double* xp, const double* nc, double (&o0)[NV], double (&o1)[NV], bool wr) {
       const size_t idx = ((size_t)row * nx + col) * NV;
       double rhs[NV];
       static_for<NV>([&](auto c) {
@@ -720,61 +750,46 @@ struct Tile {
 #pragma unroll
         for (int c = 0; c < NV; ++c) put_out(rhs[c], Out, idx + c, 0, c);
       } else {
-        // every operand of the record is loaded before the first store.  The
-        // compiler cannot prove the output distinct from the inputs (it is
-        // not, for the RK stages that update U in place), so loads
-        // interleaved with the stores would each wait for memory: six round
-        // trips per row instead of one
         const auto out = Out;
         if (sd.op == 0) {
-          double u[NV];
+          load(o0, Uin, idx, row, wr);
 #pragma unroll
-          for (int c = 0; c < NV; ++c) u[c] = operand(Uin, idx + c, row, c, wr);
-#pragma unroll
-          for (int c = 0; c < NV; ++c) put_out(u[c] + cdt * rhs[c], out, idx + c, 0, c);
+          for (int c = 0; c < NV; ++c) put_out(from(o0[c], Uin, row, c, wr) + cdt * rhs[c], out, idx + c, 0, c);
         } else if (sd.op == 2) {
           // RK104 after its fifth stage: w0 += dt/6 F (VecAXPY); w1 =
           // 1/25 U + 9/25 w0 (VecAXPBYPCZ, c = 0) into U; w0 = 15 w1 - 5 w0
           // (VecAXPBY) into A
           const auto A = Ab;
-          double u[NV], o[NV];
+          load(o0, Uin, idx, row, wr);
+          load(o1, Out, idx, row, wr);
 #pragma unroll
           for (int c = 0; c < NV; ++c) {
-            u[c] = operand(Uin, idx + c, row, c, wr);
-            o[c] = out[idx + c];
-          }
-#pragma unroll
-          for (int c = 0; c < NV; ++c) {
-            const double w0 = u[c] + cdt * rhs[c];
-            const double w1 = sd.a * o[c] + sd.g * w0;
+            const double w0 = from(o0[c], Uin, row, c, wr) + cdt * rhs[c];
+            const double w1 = sd.a * o1[c] + sd.g * w0;
             put_out(w1, out, idx + c, 0, c);
             put_out(15.0 * w1 + -5.0 * w0, A, idx + c, 1, c);
           }
         } else {
-          const auto X = Xb;
-          const auto Z = Zb;
-          double x[NV], z[NV];
+          load(o0, Xb, idx, row, wr);
+          load(o1, Zb, idx, row, wr);
 #pragma unroll
-          for (int c = 0; c < NV; ++c) {
-            x[c] = operand(X, idx + c, row, c, wr);
-            z[c] = operand(Z, idx + c, row, c, wr);
-          }
-#pragma unroll
-          for (int c = 0; c < NV; ++c) put_out(sd.a * x[c] + cdt * rhs[c] + sd.g * z[c], out, idx + c, 0, c);
+          for (int c = 0; c < NV; ++c)
+            put_out(sd.a * from(o0[c], Xb, row, c, wr) + cdt * rhs[c] + sd.g * from(o1[c], Zb, row, c, wr), out, idx + c,
+                    0, c);
         }
       }
     };
     // called by the whole wave (the flush of staged rows needs every lane)
     auto assemble = [&](int row, const double* Gt, const double* Gb, const double* Et, const double* Eb,
-                        const double* xp, const double* nc, bool wr) {
+                        const double* xp, const double* nc, double (&o0)[NV], double (&o1)[NV], bool wr) {
       if constexpr (STAGE_ROWS) {
         if (mode == HYPE_MODE_PRIME) return;
-        if (owned) record(row, Gt, Gb, Et, Eb, xp, nc, wr);
+        if (owned) record(row, Gt, Gb, Et, Eb, xp, nc, o0, o1, wr);
         flush(Out, row, 0);
         if (mode == HYPE_MODE_STAGE && sd.op == 2) flush(Ab, row, 1);
       } else {
         if (!owned || mode == HYPE_MODE_PRIME) return;
-        record(row, Gt, Gb, Et, Eb, xp, nc, wr);
+        record(row, Gt, Gb, Et, Eb, xp, nc, o0, o1, wr);
       }
     };
 
@@ -892,6 +907,11 @@ struct Tile {
         put_inlet(sn, r + 3);
       }
 
+      double o0[NV], o1[NV];
+      if constexpr (AHEAD) {
+        if (doAsm) operands(r - 1, o0, o1, true);
+      }
+
       // ---- volume non-conservative product (rhs_function_prim.c:461-479)
       double ncp[NV];
 #pragma unroll
@@ -1003,7 +1023,7 @@ struct Tile {
       }
 
       // ---- assembly + stage update of cell (col, r-1) --------------------
-      if (doAsm) assemble(r - 1, Gy, Gprev, Ey, Eprev, xpartPrev, ncpPrev, true);  // rows r-2..r+2 are in the window
+      if (doAsm) assemble(r - 1, Gy, Gprev, Ey, Eprev, xpartPrev, ncpPrev, o0, o1, true);  // rows r-2..r+2 are in the window
 
       // ---- carry -----------------------------------------------------------
 #pragma unroll
@@ -1068,7 +1088,8 @@ struct Tile {
           alo[q] = X_(0, q, NV);
           ahi[q] = X_(1, q, NV);
         }
-        double Gm[NV], Em[NV];
+        double Gm[NV], Em[NV], o0[NV], o1[NV];
+        if constexpr (AHEAD) operands(upper ? ym : ym - 1, o0, o1, false);  // row ym has left the window
         Side slo[SIDES ? NGF : 1], shi[SIDES ? NGF : 1];
         if constexpr (SIDES) {
 #pragma unroll
@@ -1079,7 +1100,7 @@ struct Tile {
         }
         yface(lo, hi, alo, ahi, slo, shi, ym, Gm, Em);
         if (!upper) {
-          assemble(ym - 1, Gm, Gprev, Em, Eprev, xpartPrev, ncpPrev, false);
+          assemble(ym - 1, Gm, Gprev, Em, Eprev, xpartPrev, ncpPrev, o0, o1, false);
         } else {
           double Gt[NV], Et[NV], xp[NV], nc[NV];
 #pragma unroll
@@ -1089,7 +1110,7 @@ struct Tile {
             xp[c] = D_(2, c);
             nc[c] = D_(3, c);
           }
-          assemble(ym, Gt, Gm, Et, Em, xp, nc, false);  // row ym has left the window
+          assemble(ym, Gt, Gm, Et, Em, xp, nc, o0, o1, false);
         }
       }
     }
