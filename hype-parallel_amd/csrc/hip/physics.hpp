@@ -76,9 +76,10 @@ struct Euler {
   static constexpr int NV = 4;
   static constexpr int WAVES_PER_EU = 2;  // register budget of the stage kernel: 256 per lane
   // tile layouts the stage kernel is built for (bit HYPE_LAYOUT_*: one wave per
-  // tile, split tiles, shared rows); the host picks per problem.  Split tiles run one wave per SIMD, one-wave tiles two: small grids gain
-  // from the shorter sweeps (256^2: 540 -> 601 Mcell-updates/s), large ones
-  // from the second wave's latency hiding
+  // tile, split tiles, shared rows); the host picks per problem.  Two-wave tiles
+  // run one wave per SIMD, one-wave tiles two: small grids gain from the shorter
+  // sweeps (256^2 at order 2, us per step: split tiles 88, shared rows 80),
+  // large ones from the second wave's latency hiding
   static constexpr int PAIR_MODES = 7;
   // a split tile sends its CFL maximum to memory once, from the lower wave,
   // instead of once per wave: the atomics of the last stage contend for one
@@ -199,8 +200,9 @@ struct Euler {
 struct Kapila {
   static constexpr int NV = 6;
   static constexpr int WAVES_PER_EU = 1;
-  // split tiles only: one reconstructed ring row per wave saved at the same
-  // one wave per SIMD (1024 x 512 shock-bubble: 952 -> 985 Mcell-updates/s)
+  // no one-wave tiles: split ones save one reconstructed ring row per wave at the
+  // same one wave per SIMD (1024 x 512 shock-bubble: 952 -> 985 Mcell-updates/s);
+  // small grids share rows (512x256: 174 -> 157 us per step)
   static constexpr int PAIR_MODES = 6;
   // one atomic per split tile (Kapila 1024x512: 1087 -> 1108
   // Mcell-updates/s; the batched set, whose 64 instances already spread the
@@ -462,8 +464,9 @@ struct Kapila {
 struct BN {
   static constexpr int NV = 9;
   static constexpr int WAVES_PER_EU = 1;
-  // one wave per tile only: two windows of nine components would halve the
-  // workgroups an LDS of 160 KB holds
+  // no split tiles: two windows of nine components would halve the workgroups an
+  // LDS of 160 KB holds.  Grids of few rows per wave share rows (128x128: 183 ->
+  // 121 us per step), which needs one window
   static constexpr int PAIR_MODES = 5;
   static constexpr bool PAIR_CFL_COMBINE = false;  // one wave per tile
   static constexpr bool HAS_INLET = false;  // no InletBC in baer_nunziato.c
