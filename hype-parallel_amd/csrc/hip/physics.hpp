@@ -425,17 +425,19 @@ struct Kapila {
     else
       B[5] = ncp5_cons(e, V, gx, gy);
   }
-  // face jump D = B(mean) (R - L) (riemann.c:95-102 / 130-137).  The products
-  // with the zero normal component add a signed zero to component 5 (or NaN, for
-  // a non-finite state: the flux's wave speed, which multiplies the jump of
-  // every component, is NaN then) and are left out.  On the primitive path the
-  // mean's factors 1/2 are kept out of the densities, where they cancel exactly
-  // (rho_k a_k^2 = (2 rho_k)(a_k^2 / 2))
+  // face jump D = B(mean) (R - L) (riemann.c:95-102 / 130-137).  On the primitive
+  // path the mean's factors 1/2 are kept out of the densities, where they cancel
+  // exactly (rho_k a_k^2 = (2 rho_k)(a_k^2 / 2)), and out of the transverse
+  // velocity, which is multiplied by zero.  Those products stay, as the zero's sign
+  // does not reach a sum but a NaN does: where a transverse velocity is not finite
+  // (its reconstruction overflows before any other component's does) the
+  // reference's jump is NaN, also where the face's wave speed is not (PetscMax
+  // keeps a left speed beside a right one that is NaN)
   template <bool PRIM, int DIR>
   __device__ static __forceinline__ void ncp_face(const Eos& e, const double* L, const double* R, double* D) {
     for (int c = 0; c < 5; ++c) D[c] = 0.0;
     if (PRIM) {
-      constexpr int n = 2 + DIR;
+      constexpr int n = 2 + DIR, t = 3 - DIR;
       double r1 = R[0] + L[0];  // twice the means
       double r2 = R[1] + L[1];
       double un = 0.5 * (R[n] + L[n]);
@@ -446,7 +448,7 @@ struct Kapila {
       double a_1_sq = fdiv(e.g1 * fma(0.5, ps, e.p1), r1);  // half of them
       double a_2_sq = fdiv(e.g2 * fma(0.5, ps, e.p2), r2);
       double K = fdiv(alpha_1 * alpha_2 * (r2 * a_2_sq - r1 * a_1_sq), alpha_1 * r2 * a_2_sq + alpha_2 * r1 * a_1_sq);
-      D[5] = un * (R[5] - L[5]) - K * (R[n] - L[n]);
+      D[5] = fma(R[t] + L[t], 0.0, un * (R[5] - L[5])) - K * fma(R[t] - L[t], 0.0, R[n] - L[n]);
     } else {
       constexpr double nx = DIR == 0 ? 1.0 : 0.0, ny = DIR == 0 ? 0.0 : 1.0;
       double av[NV], gx[NV], gy[NV];
