@@ -286,7 +286,7 @@ struct Duo {
       const size_t idx = ((size_t)row * nx + col) * NV;
       double rhs[NV];
       static_for<NV>([&](auto c) {
-        const double t = P_(c) - T1::template face_diff<1, c>(r1_h, Gt[c], Gb[c], Et[c], Eb[c]);
+        const double t = P_(c) - T1::template face_diff<c>(r1_h, Gt[c], Gb[c], Et[c], Eb[c]);
         rhs[c] = ((S::HAS_NCP && S::DNZ[c]) ? P_(NV + jump_index(c)) : 0.0) + t;
       });
       if (mode == HYPE_MODE_RHS) {
@@ -364,7 +364,7 @@ struct Duo {
         if constexpr (CHECK_EACH) {
           if (__builtin_expect(__ballot(bad[q]) != 0, 0)) report(key0, q, Lv[q], Rv[q], mine, bad[q]);
         }
-        T1::template add_point<DIR>(q, A, D, G, E);
+        T1::add_point(q, A, D, G, E);
       }
       if (!CHECK_EACH && __builtin_expect(__ballot(any) != 0, 0)) {
 #pragma unroll
@@ -549,9 +549,8 @@ struct Duo {
                   double V[NV], gx[NV], gy[NV], B[NV];
                   T1::template at_vol<q>(co, r1_h, V, gx, gy);
                   S::template vol_ncp<PRIM>(eos, V, gx, gy, B);
-                  T1::template add_volume<q>(B, ncp);
+                  T1::add_volume(B, ncp);
                 });
-                T1::scale_volume(ncp);
                 static_for<NV>([&](auto c) {
                   if constexpr (S::DNZ[c]) keep[NV + jump_index(c)] = ncp[c];
                 });
@@ -573,7 +572,7 @@ struct Duo {
             face(std::integral_constant<int, 0>{}, vl, lv, ls, lo, ((long)r * (nx + 1) + col) * NGF, xlane, Fx, Dx);
             static_for<NV>([&](auto c) {
               const double Dr = S::DNZ[c] ? lane_from_right(Dx[c]) : 0.0;
-              keep[c] = -T1::template face_diff<0, c>(r1_h, lane_from_right(Fx[c]), Fx[c], Dr, Dx[c]);
+              keep[c] = -T1::template face_diff<c>(r1_h, lane_from_right(Fx[c]), Fx[c], Dr, Dx[c]);
             });
           }
         } else {

@@ -11,15 +11,13 @@
 // The stage kernel is bound by the number of FP64 instructions, so where the
 // reference multiplies by a power of two or by zero (an exact product) and adds,
 // the two are one fused multiply-add here: it rounds once, to the same bits.
-// With the constant denominators' reciprocals, the face sums' weights folded into
-// the assembly and the admissibility report off the common path, a Kapila row's
-// faces take 810 FP64 instructions instead of 1,240 (1024x512, 10 SSP-RK steps:
-// 4503 -> 4247 us; Baer-Nunziato 2048x1024, 3 steps: 8647 -> 8191 us; Euler
-// 256x256, 20 steps: 1934 -> 1834 us).
+// With the constant denominators' reciprocals and the admissibility report off the
+// common path, a Kapila row's faces take 860 FP64 instructions instead of 1,240.
 // Halving is exact except for subnormal numbers.  Velocities and momenta do get
 // there: ahead of a wave they decay by a factor per cell down to the smallest
-// doubles.  S::TINY marks those components and S::JUMP_TINY those whose jump term
-// is a product with one; their sums keep the reference's separate operations.
+// doubles.  S::TINY marks those components, whose sums keep the reference's
+// separate operations; so do the fluxes and jump terms of every component, which
+// are products with a velocity.
 // Densities, energies, pressures and volume fractions are normal numbers, and so
 // are their differences (zero or at least an ulp).
 #pragma once
@@ -97,7 +95,6 @@ struct Euler {
   // components of the flux that are identically zero
   static constexpr bool FZERO[NV] = {false, false, false, false};
   static constexpr bool TINY[NV] = {false, true, true, false};
-  static constexpr bool JUMP_TINY[NV] = {false, false, false, false};
   __device__ static __forceinline__ void energy_den(const Eos& e, double& d1, double& d2) {
     d1 = e.g1 - 1.0;
     d2 = 1.0;
@@ -221,7 +218,6 @@ struct Kapila {
 
   static constexpr bool FZERO[NV] = {false, false, false, false, false, true};
   static constexpr bool TINY[NV] = {false, false, true, true, false, false};
-  static constexpr bool JUMP_TINY[NV] = {false, false, false, false, false, true};
   __device__ static __forceinline__ void energy_den(const Eos& e, double& d1, double& d2) {
     d1 = (e.g1 - 1.0) * (e.g2 - 1.0);
     d2 = 1.0;
@@ -481,7 +477,6 @@ struct BN {
 
   static constexpr bool FZERO[NV] = {false, false, false, false, false, false, false, false, true};
   static constexpr bool TINY[NV] = {false, true, true, false, false, true, true, false, false};
-  static constexpr bool JUMP_TINY[NV] = {false, false, false, false, false, false, false, false, false};
   __device__ static __forceinline__ void energy_den(const Eos& e, double& d1, double& d2) {
     d1 = e.g1 - 1.0;
     d2 = e.g2 - 1.0;
