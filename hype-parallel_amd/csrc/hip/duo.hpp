@@ -64,7 +64,7 @@ struct Duo {
   __device__ static __forceinline__ void at_nodes(const double (&co)[NV][NDOF], double (&fv)[NN][NV]) {
     static_for<NN>([&](auto i) {
       static_for<NV>([&](auto c) {
-        fv[i][c] = basis_sum<RowNode<N, (X ? 0 : 2 * NGF) + i>, NDOF, S::TINY[c]>(co[c]);
+        fv[i][c] = basis_sum<RowNode<N, (X ? 0 : 2 * NGF) + i>, NDOF, S::RANGE[PRIM][c] != NORMAL>(co[c]);
       });
     });
   }
@@ -438,7 +438,7 @@ struct Duo {
             ud[2] = W_(sm1, c, cw + 1);
             ud[3] = W_(sp1, c, cw - 1);
             ud[4] = W_(sm1, c, cw - 1);
-            reconstruct<N, S::TINY[c]>(ux, uy, ud, co[c]);
+            reconstruct<N, S::RANGE[PRIM][c]>(ux, uy, ud, co[c]);
 #pragma unroll
             for (int k = 1; k < NDOF; ++k) C_(c, k) = co[c][k];
           }

@@ -15,11 +15,15 @@
 // common path, a Kapila row's faces take 860 FP64 instructions instead of 1,240.
 // Halving is exact except for subnormal numbers.  Velocities and momenta do get
 // there: ahead of a wave they decay by a factor per cell down to the smallest
-// doubles.  S::TINY marks those components, whose sums keep the reference's
-// separate operations; so do the fluxes and jump terms of every component, which
-// are products with a velocity.
-// Densities, energies, pressures and volume fractions are normal numbers, and so
-// are their differences (zero or at least an ulp).
+// doubles.  So does the first phase's volume fraction where that phase vanishes,
+// and its mass, momentum and energy per volume with it (the second phase's is one
+// minus the first's).  S::RANGE names those components of the conservative [0] and
+// the primitive [1] path; their sums keep the reference's separate operations.  So
+// do the fluxes and jump terms of every component, which are products with a
+// velocity.
+// The other components, densities, pressures and the energies with them, are
+// bounded from below by the admissibility checks, so they and their differences
+// (zero or at least an ulp) are normal numbers.
 #pragma once
 #ifndef HYPE_KNS
 #define HYPE_KNS hype  // kernel namespace; the contracted build uses its own
@@ -34,6 +38,10 @@ namespace HYPE_KNS {
 constexpr double PRS_FLOOR = 1.0e-12;
 constexpr double RHO_FLOOR = 1.0e-14;
 constexpr double SMALL_NUM = 1.0e-12;
+
+// which numbers a component takes: normal ones and zero, any of either sign, or
+// any positive one
+enum Range { NORMAL, ANY, POSITIVE };
 
 struct Eos {
   double g1, g2, p1, p2;  // GAMMA_1, GAMMA_2, PI_1, PI_2 (hype.h:42-45)
@@ -94,7 +102,7 @@ struct Euler {
 
   // components of the flux that are identically zero
   static constexpr bool FZERO[NV] = {false, false, false, false};
-  static constexpr bool TINY[NV] = {false, true, true, false};
+  static constexpr Range RANGE[2][NV] = {{NORMAL, ANY, ANY, NORMAL}, {NORMAL, ANY, ANY, NORMAL}};
   __device__ static __forceinline__ void energy_den(const Eos& e, double& d1, double& d2) {
     d1 = e.g1 - 1.0;
     d2 = 1.0;
@@ -217,7 +225,8 @@ struct Kapila {
   static constexpr bool DNZ[NV] = {false, false, false, false, false, true};
 
   static constexpr bool FZERO[NV] = {false, false, false, false, false, true};
-  static constexpr bool TINY[NV] = {false, false, true, true, false, false};
+  static constexpr Range RANGE[2][NV] = {{POSITIVE, NORMAL, ANY, ANY, NORMAL, POSITIVE},
+                                         {NORMAL, NORMAL, ANY, ANY, NORMAL, POSITIVE}};
   __device__ static __forceinline__ void energy_den(const Eos& e, double& d1, double& d2) {
     d1 = (e.g1 - 1.0) * (e.g2 - 1.0);
     d2 = 1.0;
@@ -476,7 +485,8 @@ struct BN {
   static constexpr bool DNZ[NV] = {false, true, true, true, false, true, true, true, true};
 
   static constexpr bool FZERO[NV] = {false, false, false, false, false, false, false, false, true};
-  static constexpr bool TINY[NV] = {false, true, true, false, false, true, true, false, false};
+  static constexpr Range RANGE[2][NV] = {{POSITIVE, ANY, ANY, POSITIVE, NORMAL, ANY, ANY, NORMAL, POSITIVE},
+                                         {NORMAL, ANY, ANY, NORMAL, NORMAL, ANY, ANY, NORMAL, POSITIVE}};
   __device__ static __forceinline__ void energy_den(const Eos& e, double& d1, double& d2) {
     d1 = e.g1 - 1.0;
     d2 = e.g2 - 1.0;

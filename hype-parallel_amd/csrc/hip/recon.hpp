@@ -17,6 +17,7 @@
 #include <utility>
 
 #include "fdiv.hpp"
+#include "physics.hpp"
 
 namespace HYPE_KNS {
 
@@ -110,7 +111,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 // sum_k s[k]*phi(k) in the reference's order, skipping exact-zero phi; T::at(k)
 // is the table row.  A product with a power of two is exact, so fusing it with
 // the addition rounds once, as the separate operations do, in one instruction.
-// TINY: the component may hold subnormal values (S::TINY), whose halves round
+// TINY: the component may hold subnormal values (S::RANGE), whose halves round
 template <class T, int NDOF, bool TINY>
 __device__ __forceinline__ double basis_sum(const double* s) {
   double acc = 0.0;
@@ -156,7 +157,7 @@ __device__ __forceinline__ double pow4(double a) {  // reconstruction.c:123-127
 // smoothness terms are then 4 times, their fourth powers 256 times the
 // reference's, which cancels in the weights; dividing by twice the weights' sum
 // undoes the doubling.
-// TINY: the component may hold subnormal values (S::TINY), whose products with
+// TINY: the component may hold subnormal values, whose products with
 // 1/2 round; the candidates then keep the reference's halves (17 operations).
 // The smoothness terms may still use the doubled curvatures: below 1e-28 they
 // vanish beside the 1e-12 they are added to.
@@ -210,12 +211,25 @@ __device__ __forceinline__ void weno3_dir(double m2, double m1, double u0, doubl
 // unscaled candidates, two Newton steps per reciprocal and FP64 range checks).  Measured over an SSP-RK
 // solve: Kapila 1024x512 4802 -> 4503 us per 10 steps, Baer-Nunziato 2048x1024
 // 9191 -> 8647 us per 3, Euler 256x256 2007 -> 1934 us per 20.
-template <bool TINY>
+//
+// A positive component (RANGE POSITIVE) is subnormal only where a phase vanishes.
+// Its doubled candidates are exact wherever the cell's own value is far above the
+// subnormal numbers: every candidate but the central slope contains that value, in
+// whose sum a subnormal neighbour's rounded half is lost, and the central slope's
+// is lost in the sum of the three.  Elsewhere (below 2^-800, or not positive, or
+// beyond 2^610) the cell is left to the plain form too: two integer operations
+// instead of weno3_dir<TINY>'s ten FP64 ones (Kapila 1024x512, 10 steps: 4136 and
+// 4043 us; 48 Kapila grids 14955 and 14637).
+constexpr unsigned POSITIVE_LOW_WORD = (1023u - 800u) << 20;  // high word of 2^-800
+
+template <Range RANGE>
 __device__ __forceinline__ bool weno3_fast(const double* U_x, const double* U_y, const double* U_xy,
                                            double* coeffs) {
+  constexpr bool TINY = RANGE == ANY;
   const double u_0 = U_xy[0];
   const double h0 = (TINY ? 1.5 : 3.0) * u_0;
-  unsigned top = 0;
+  // wraps below 2^-800 to more than FDIV_TOP_WORD
+  unsigned top = RANGE == POSITIVE ? hi_word(u_0) - POSITIVE_LOW_WORD : 0;
   double c1, c2, c3, c4;
   weno3_dir<TINY>(U_x[0], U_x[1], u_0, U_x[3], U_x[4], h0, c1, c3, top);
   weno3_dir<TINY>(U_y[0], U_y[1], u_0, U_y[3], U_y[4], h0, c2, c4, top);
@@ -362,7 +376,7 @@ __device__ __forceinline__ bool weno4(const double* U_x, const double* U_y, cons
 // Stencil of one component: x[0..4] = u(i-2..i+2, j), y[0..4] = u(i, j-2..j+2),
 // d[0..4] = u(i,j), u(i+1,j+1), u(i+1,j-1), u(i-1,j+1), u(i-1,j-1)
 // (rhs_function_prim.c:332-348).
-template <int N, bool TINY>
+template <int N, Range RANGE>
 __device__ __forceinline__ void reconstruct(const double* U_x, const double* U_y, const double* U_xy,
                                             double* coeffs) {
   if constexpr (N == 0) {
@@ -374,9 +388,10 @@ __device__ __forceinline__ void reconstruct(const double* U_x, const double* U_y
     coeffs[1] = minmod(U_x[3] - u_0, u_0 - U_x[1]);
     coeffs[2] = minmod(U_y[3] - u_0, u_0 - U_y[1]);
   } else if constexpr (N == 3) {
+    constexpr bool TINY = RANGE != NORMAL;
     if (!__builtin_expect((weno4<true, TINY>(U_x, U_y, U_xy, coeffs)), 1)) weno4<false, TINY>(U_x, U_y, U_xy, coeffs);
   } else {
-    if (__builtin_expect(weno3_fast<TINY>(U_x, U_y, U_xy, coeffs), 1)) return;
+    if (__builtin_expect(weno3_fast<RANGE>(U_x, U_y, U_xy, coeffs), 1)) return;
     // reconstruction.c:144-221
     const double central_cell_wt = 100.0;
     const double r13_3 = 13. / 3.;

@@ -362,7 +362,7 @@ struct Tile {
   // (rhs_function_prim.c:382-388, 425-440)
   __device__ static __forceinline__ void at_nodes(const double (&co)[NV][NDOF], double (&fv)[NNODE][NV]) {
     static_for<NNODE>([&](auto P) {
-      static_for<NV>([&](auto c) { fv[P][c] = basis_sum<RowNode<N, P>, NDOF, S::TINY[c]>(co[c]); });
+      static_for<NV>([&](auto c) { fv[P][c] = basis_sum<RowNode<N, P>, NDOF, S::RANGE[PRIM][c] != NORMAL>(co[c]); });
     });
   }
   // value and scaled gradient at volume point q (rhs_function_prim.c:442-455)
@@ -370,9 +370,9 @@ struct Tile {
   __device__ static __forceinline__ void at_vol(const double (&co)[NV][NDOF], double r1_h, double* V, double* gx,
                                                 double* gy) {
     static_for<NV>([&](auto c) {
-      V[c] = basis_sum<RowVol<N, q>, NDOF, S::TINY[c]>(co[c]);
-      gx[c] = r1_h * basis_sum<RowGx<N, q>, NDOF, S::TINY[c]>(co[c]);
-      gy[c] = r1_h * basis_sum<RowGy<N, q>, NDOF, S::TINY[c]>(co[c]);
+      V[c] = basis_sum<RowVol<N, q>, NDOF, S::RANGE[PRIM][c] != NORMAL>(co[c]);
+      gx[c] = r1_h * basis_sum<RowGx<N, q>, NDOF, S::RANGE[PRIM][c] != NORMAL>(co[c]);
+      gy[c] = r1_h * basis_sum<RowGy<N, q>, NDOF, S::RANGE[PRIM][c] != NORMAL>(co[c]);
     });
   }
 
@@ -820,7 +820,7 @@ struct Tile {
         ud[2] = W_(sm1, c, cw + 1);
         ud[3] = W_(sp1, c, cw - 1);
         ud[4] = W_(sm1, c, cw - 1);
-        reconstruct<N, S::TINY[c]>(ux, uy, ud, co[c]);
+        reconstruct<N, S::RANGE[PRIM][c]>(ux, uy, ud, co[c]);
       });
       // values at the nodes, which are also the face quadrature points
       // (rhs_function_prim.c:382-388, 425-440; the same points, hype.c:207-229)
