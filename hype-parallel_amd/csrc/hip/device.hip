@@ -175,7 +175,8 @@ int hyped_blocks_per_cu(const hype_variant* v) { return v->fma ? hype_fc::blocks
 
 int hyped_block_waves(const hype_variant* v) { return v->pair ? 2 : 1; }
 
-int hyped_pair_modes(int system, int order) { return hype::pair_modes(system, order); }  // the same in both builds
+// of the exact build; hype_layouts leaves out what the contracted one lacks
+int hyped_pair_modes(int system, int order) { return hype::pair_modes(system, order); }
 
 int hyped_graph_begin(void* s) {
   HCHECK(hipStreamBeginCapture((hipStream_t)s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");

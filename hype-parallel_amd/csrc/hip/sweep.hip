@@ -1189,7 +1189,7 @@ __global__ __launch_bounds__(LAY ? 2 * HYPE_WAVE : HYPE_WAVE)
 template <class S, int N>
 static constexpr int layouts() {
 #if defined(HYPE_CONTRACTED_BUILD)
-  return S::PAIR_MODES & 3;  // its solves use the layouts of batches (hype_layouts)
+  return S::PAIR_MODES & 3;  // no shared rows (hype_layouts leaves them out)
 #else
   return N == 2 || (N == 3 && S::NV <= 6) ? S::PAIR_MODES : S::PAIR_MODES & 3;
 #endif

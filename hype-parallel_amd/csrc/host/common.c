@@ -180,14 +180,13 @@ void hype_decode_error(unsigned long long word, int nx, int ny, int ngf,
     snprintf(msg, cap, "%s\nAt x = %f, y = %f", head, *x, *y);
 }
 
-/* tile layouts (bits HYPE_LAYOUT_*) a problem may use: those the system's kernel is built for, narrowed by the layout bits
- * of its options */
+/* tile layouts (bits HYPE_LAYOUT_*) a problem may use: those the system's exact
+ * kernel is built for, narrowed by the bits of its options */
 int hype_layouts(const hype_problem *p, int built)
 {
     if (p->options & HYPE_OPT_ONE_WAVE_TILES) return built & 1;
     if (p->options & HYPE_OPT_SPLIT_TILES) return built & 2;
-    /* contraction differs between the layouts' kernels: a contracted solve keeps
-     * to those of batches and servers, whose results it must match */
+    /* the contracted build has no shared-row kernels */
     if (p->options & HYPE_OPT_FMA) return built & 3;
     return built;
 }

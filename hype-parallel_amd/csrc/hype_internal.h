@@ -158,8 +158,8 @@ int hyped_num_cus(void);
 int hyped_blocks_per_cu(const hype_variant *v);
 /* waves per workgroup of that kernel: 1 with one wave per tile, else 2 */
 int hyped_block_waves(const hype_variant *v);
-/* tile layouts (bits HYPE_LAYOUT_*) a system's stage kernel of an order is built
- * for */
+/* tile layouts (bits HYPE_LAYOUT_*) a system's exact stage kernel of an order is
+ * built for; the contracted one lacks shared rows */
 int hyped_pair_modes(int system, int order);
 const char *hyped_last_error(void);
 /* this device's address of the scratch array and its size (looked up on the

@@ -80,8 +80,9 @@ typedef struct hype_problem {
 } hype_problem;
 
 /* ---- numerics options --------------------------------------------------- */
-/* Run the kernels built with FMA contraction: a*b+c fused wherever the
- * compiler can (about 10 % faster on MI355X).  Results stay within the
+/* Run the kernels built with FMA contraction: a*b+c fused within an
+ * expression (up to 6 % faster on MI355X; slower on small grids at orders 2 and
+ * 3, where the exact kernels share rows).  Results stay within the
  * FP64 tolerances of the reference path (relative 1e-12 per RHS evaluation)
  * but are no longer bitwise equal to the uncontracted arithmetic; a
  * threshold decision on a value within rounding of it (admissibility, WENO
@@ -98,7 +99,8 @@ typedef struct hype_problem {
  * grid fills two waves per SIMD), and batches and servers use split tiles
  * for Kapila and one wave per tile otherwise.  These bits force a layout; one
  * the system's kernel is not built for is HYPE_E_UNSUPPORTED.  Results are
- * bitwise the same either way. */
+ * bitwise the same either way, with HYPE_OPT_FMA too (whose kernels are not
+ * built for shared rows). */
 #define HYPE_OPT_ONE_WAVE_TILES 0x2u
 #define HYPE_OPT_SPLIT_TILES 0x4u
 
