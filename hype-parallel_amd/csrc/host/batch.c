@@ -217,23 +217,31 @@ int hype_batch_tiling(hype_batch *b, int *rows, int *tiles, int *groups)
     return HYPE_OK;
 }
 
+static int set_plan(hype_batch *b, int rows, int by_time)
+{
+    HYPE_TRY(by_time ? eng_set_rows_by_time(&b->E, rows) : eng_set_rows(&b->E, rows));
+    return eng_commit(&b->E);
+}
+
 int hype_batch_set_rows(hype_batch *b, int rows)
 {
     if (!b) return HYPE_E_INVALID;
-    HYPE_TRY(eng_set_rows(&b->E, rows));
-    return eng_commit(&b->E);
+    return set_plan(b, rows, 0);
 }
 
 /* Measured tuning of the tile shape and LDS footprint: time `steps` steps
  * of every candidate tile height, and, where an instance's system is built
  * for both tile layouts (one wave per tile with one LDS window, or tiles
  * split over two waves with two windows and the exchange areas), of both
- * layouts; keep the fastest pair.  The states are advanced from the current
+ * layouts; keep the fastest plan.  Where the instances' rows take different
+ * times, a candidate is timed as every instance's height and as that of the
+ * instances with the quickest rows, the others' lower by their row time, as in
+ * the automatic plan (eng_auto_rows).  The states are advanced from the current
  * ones: set them again afterwards. */
 int hype_batch_autotune(hype_batch *b, const int *cand, int ncand, int steps, int *best_rows,
                         double *best_ms)
 {
-    int k, i, l, best = -1, best_layout = -1, nlay = 1, rc = HYPE_OK;
+    int k, i, l, w, best = -1, best_w = 0, best_layout = -1, nlay = 1, rc = HYPE_OK;
     int layouts[2] = {-1, 1};
     double bms = 1e300;
     double *t_end;
@@ -254,18 +262,21 @@ int hype_batch_autotune(hype_batch *b, const int *cand, int ncand, int steps, in
     }
     for (l = 0; l < nlay && rc == HYPE_OK; ++l) {
         if ((rc = eng_set_layout(&b->E, layouts[l])) != HYPE_OK) break;
-        for (k = 0; k < ncand; ++k) {
-            double ms = 0.0;
+        for (k = 0; k < ncand && rc == HYPE_OK; ++k) {
             if (cand[k] < 1) continue;
-            if ((rc = hype_batch_set_rows(b, cand[k])) != HYPE_OK ||
-                (rc = hype_batch_begin(b, NULL, t_end, maxs, 0)) != HYPE_OK ||
-                (rc = hype_batch_advance(b, 1)) != HYPE_OK ||
-                (rc = hype_batch_advance_timed(b, steps, &ms)) != HYPE_OK)
-                break;
-            if (ms < bms) {
-                bms = ms;
-                best = cand[k];
-                best_layout = layouts[l];
+            for (w = 0; w <= eng_mixed(&b->E, NULL); ++w) {
+                double ms = 0.0;
+                if ((rc = set_plan(b, cand[k], w)) != HYPE_OK ||
+                    (rc = hype_batch_begin(b, NULL, t_end, maxs, 0)) != HYPE_OK ||
+                    (rc = hype_batch_advance(b, 1)) != HYPE_OK ||
+                    (rc = hype_batch_advance_timed(b, steps, &ms)) != HYPE_OK)
+                    break;
+                if (ms < bms) {
+                    bms = ms;
+                    best = cand[k];
+                    best_w = w;
+                    best_layout = layouts[l];
+                }
             }
         }
     }
@@ -276,7 +287,7 @@ int hype_batch_autotune(hype_batch *b, const int *cand, int ncand, int steps, in
     if (best_rows) *best_rows = best;
     if (best_ms) *best_ms = bms;
     HYPE_TRY(eng_set_layout(&b->E, best_layout));
-    return hype_batch_set_rows(b, best);
+    return set_plan(b, best, best_w);
 }
 
 int hype_batch_layout(hype_batch *b, int *layout)

@@ -327,6 +327,25 @@ int eng_pick_rows(hype_engine *E)
     return best;
 }
 
+/* 1 if the running slots' tile rows take different times; *lo (may be NULL): the
+ * least of them.  The line lies between Euler's one-wave and Kapila's split tiles
+ * (1.08), for which one height and its model of whole rounds of tiles serve, and
+ * order 3 beside order 2 (1.3). */
+int eng_mixed(const hype_engine *E, double *lo)
+{
+    double min = 1e300, max = 0.0;
+    int s;
+    for (s = 0; s < E->cap; ++s) {
+        double t;
+        if (!E->used[s] || !E->run[s]) continue;
+        t = tile_row_time(E, s);
+        if (t < min) min = t;
+        if (t > max) max = t;
+    }
+    if (lo) *lo = min;
+    return max > 1.25 * min;
+}
+
 /* Heights for a mix of systems.  A Baer-Nunziato row takes three times as long as
  * an Euler row, and the groups' launches run side by side, so one height for all
  * leaves a stage waiting for a few tall Baer-Nunziato tiles while the rest of the
@@ -337,16 +356,9 @@ int eng_pick_rows(hype_engine *E)
 int eng_auto_rows(hype_engine *E)
 {
     const double simds = 4.0 * E->ncu;
-    double lo = 1e300, hi = 0.0, best_t = 1e300;
+    double lo, best_t = 1e300;
     int s, h, best = 1;
-    for (s = 0; s < E->cap; ++s) {
-        double t;
-        if (!E->used[s] || !E->run[s]) continue;
-        t = tile_row_time(E, s);
-        if (t < lo) lo = t;
-        if (t > hi) hi = t;
-    }
-    if (hi <= 1.25 * lo) return eng_set_rows(E, eng_pick_rows(E));
+    if (!eng_mixed(E, &lo)) return eng_set_rows(E, eng_pick_rows(E));
     for (h = 1; h <= 256; ++h) {
         double work = 0.0, tail = 0.0;
         for (s = 0; s < E->cap; ++s) {
@@ -364,10 +376,7 @@ int eng_auto_rows(hype_engine *E)
             best = h;
         }
     }
-    E->target_rows = best;
-    E->weighted = 1;
-    E->row_min = lo;
-    return HYPE_OK;
+    return eng_set_rows_by_time(E, best);
 }
 
 int eng_set_rows(hype_engine *E, int rows)
@@ -375,6 +384,14 @@ int eng_set_rows(hype_engine *E, int rows)
     if (rows < 1) return HYPE_E_INVALID;
     E->target_rows = rows;
     E->weighted = 0;
+    return HYPE_OK;
+}
+
+int eng_set_rows_by_time(hype_engine *E, int rows)
+{
+    HYPE_TRY(eng_set_rows(E, rows));
+    eng_mixed(E, &E->row_min);
+    E->weighted = 1;
     return HYPE_OK;
 }
 

@@ -101,7 +101,11 @@ int eng_pick_rows(hype_engine *E);
 /* set the tile heights the model picks for the running slots: common, or by
  * system where their rows take different times */
 int eng_auto_rows(hype_engine *E);
+int eng_mixed(const hype_engine *E, double *lo);
+/* one height for all slots, or one for those whose rows take the least time and
+ * the others in inverse proportion */
 int eng_set_rows(hype_engine *E, int rows);
+int eng_set_rows_by_time(hype_engine *E, int rows);
 int eng_total_tiles(hype_engine *E);
 
 #endif

@@ -308,13 +308,19 @@ int hype_batch_advance_timed(hype_batch *b, int nsteps, double *ms);
  * described by hype_batch_last_error) */
 int hype_batch_sync(hype_batch *b, hype_status *st);
 const char *hype_batch_last_error(hype_batch *b, double *x, double *y);
+/* *rows: tile height of every instance, or, in a plan with heights by system (the
+ * automatic plan of a mix of systems or orders whose rows take different times,
+ * or what hype_batch_autotune left), of those with the quickest rows; the others'
+ * are lower by their row time.  hype_batch_set_rows gives all instances one
+ * height. */
 int hype_batch_tiling(hype_batch *b, int *rows, int *tiles, int *groups);
 int hype_batch_set_rows(hype_batch *b, int rows);
 /* Measured tuning of the tile shape and LDS footprint: times `steps` steps
  * at every candidate tile height and, where an instance's system is built
  * for both tile layouts (one wave per tile with one LDS window, or each
  * tile split over a two-wave workgroup with two windows and exchange
- * areas: Euler), in both layouts, and keeps the fastest pair.  Advances the
+ * areas: Euler), in both layouts; in a mix whose rows take different times each
+ * height also with heights by system.  Keeps the fastest plan.  Advances the
  * current states: set them again afterwards. */
 int hype_batch_autotune(hype_batch *b, const int *cand, int ncand, int steps,
                         int *best_rows, double *best_ms);
