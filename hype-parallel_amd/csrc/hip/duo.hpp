@@ -56,7 +56,8 @@ struct Duo {
   static constexpr int COF = NV * (NDOF - 1) * HYPE_WAVE;
   static constexpr int PART = (NV + njump()) * HYPE_WAVE;
   static constexpr int XST = PRIM ? 16 * 4 * NV : 0;
-  static constexpr int OST = STAGE_ROWS ? (N == 3 ? 2 : 1) * NV * HYPE_TILE_W : 0;
+  static_assert(!(STAGE_ROWS && N == 3), "RK104's second output row is not staged: layouts() leaves this out");
+  static constexpr int OST = STAGE_ROWS ? NV * HYPE_TILE_W : 0;
   static constexpr int LDS = WIN + COF + PART + XST + OST + 3;
 
   // values of all components at the wave's nodes
@@ -265,15 +266,14 @@ struct Duo {
     };
 
     // ---- output (as in Tile) --------------------------------------------
-    auto put_out = [&](double val, gmem_t<double>* dst, size_t i, int k, int c) {
-      if constexpr (STAGE_ROWS) ost[(k * HYPE_TILE_W + lane - 1) * NV + c] = val;
+    auto put_out = [&](double val, gmem_t<double>* dst, size_t i, int c) {
+      if constexpr (STAGE_ROWS) ost[(lane - 1) * NV + c] = val;
       else __builtin_nontemporal_store(val, &dst[i]);
     };
-    auto flush = [&](gmem_t<double>* dst, int row, int k) {
+    auto flush = [&](gmem_t<double>* dst, int row) {
       wave_sync();
       const size_t first = ((size_t)row * nx + x0) * NV;
-      const double* src = ost + k * HYPE_TILE_W * NV;
-      for (int e = lane; e < W * NV; e += HYPE_WAVE) __builtin_nontemporal_store(src[e], &dst[first + e]);
+      for (int e = lane; e < W * NV; e += HYPE_WAVE) __builtin_nontemporal_store(ost[e], &dst[first + e]);
       wave_sync();
     };
     auto operand = [&](gmem_t<const double>* B, size_t i, int row, int c) -> double {
@@ -291,13 +291,13 @@ struct Duo {
       });
       if (mode == HYPE_MODE_RHS) {
 #pragma unroll
-        for (int c = 0; c < NV; ++c) put_out(rhs[c], Out, idx + c, 0, c);
+        for (int c = 0; c < NV; ++c) put_out(rhs[c], Out, idx + c, c);
       } else if (sd.op == 0) {
         double u[NV];
 #pragma unroll
         for (int c = 0; c < NV; ++c) u[c] = operand(Uin, idx + c, row, c);
 #pragma unroll
-        for (int c = 0; c < NV; ++c) put_out(u[c] + cdt * rhs[c], Out, idx + c, 0, c);
+        for (int c = 0; c < NV; ++c) put_out(u[c] + cdt * rhs[c], Out, idx + c, c);
       } else if (sd.op == 2) {
         if constexpr (N == 3) {  // RK104 after its fifth stage
           double u[NV], o[NV];
@@ -310,8 +310,8 @@ struct Duo {
           for (int c = 0; c < NV; ++c) {
             const double w0 = u[c] + cdt * rhs[c];
             const double w1 = sd.a * o[c] + sd.g * w0;
-            put_out(w1, Out, idx + c, 0, c);
-            put_out(15.0 * w1 + -5.0 * w0, Ab, idx + c, 1, c);
+            put_out(w1, Out, idx + c, c);
+            put_out(15.0 * w1 + -5.0 * w0, Ab, idx + c, c);
           }
         }
       } else {
@@ -322,15 +322,14 @@ struct Duo {
           z[c] = operand(Zb, idx + c, row, c);
         }
 #pragma unroll
-        for (int c = 0; c < NV; ++c) put_out(sd.a * x[c] + cdt * rhs[c] + sd.g * z[c], Out, idx + c, 0, c);
+        for (int c = 0; c < NV; ++c) put_out(sd.a * x[c] + cdt * rhs[c] + sd.g * z[c], Out, idx + c, c);
       }
     };
     auto assemble = [&](int row, const double* Gt, const double* Gb, const double* Et, const double* Eb) {
       if (mode == HYPE_MODE_PRIME) return;
       if (owned) record(row, Gt, Gb, Et, Eb);
       if constexpr (STAGE_ROWS) {
-        flush(Out, row, 0);
-        if (N == 3 && mode == HYPE_MODE_STAGE && sd.op == 2) flush(Ab, row, 1);
+        flush(Out, row);
       }
     };
 

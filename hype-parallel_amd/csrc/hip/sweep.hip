@@ -1075,15 +1075,7 @@ struct Tile {
         }
         double Gm[NV], Em[NV], o0[NV], o1[NV];
         if constexpr (AHEAD) operands(upper ? ym : ym - 1, o0, o1, false);  // row ym has left the window
-        Side slo[SIDES ? NGF : 1], shi[SIDES ? NGF : 1];
-        if constexpr (SIDES) {
-#pragma unroll
-          for (int q = 0; q < NGF; ++q) {
-            slo[q].template of<1>(eos, lo[q]);
-            shi[q].template of<1>(eos, hi[q]);
-          }
-        }
-        yface(lo, hi, alo, ahi, slo, shi, ym, Gm, Em);
+        yface(lo, hi, alo, ahi, nullptr, nullptr, ym, Gm, Em);  // no SIDES in split tiles
         if (!upper) {
           assemble(ym - 1, Gm, Gprev, Em, Eprev, xpartPrev, ncpPrev, o0, o1, false);
         } else {
