@@ -45,8 +45,12 @@ __device__ __forceinline__ unsigned hi_word(double x) { return (unsigned)__doubl
 // e = 1 - b y0, in place of the sequence's two Newton steps: three fused
 // operations instead of four.  |e| <= 2^-23 (the hardware's bound for
 // v_rcp_f64), so the step's own error is below 2^-68 and the result is the
-// rounded reciprocal up to 2^-15 of an ulp in the halfway cases, as the
-// quotient and remainder step below need it
+// rounded reciprocal up to 2^-15 of an ulp in the halfway cases.  The sequence's
+// is so up to 2^-39: that the quotient and remainder step below round correctly
+// from either is an observation.  On the device none of 5.4e8 quotients and as
+// many reciprocals differed from the compiler's (a quarter of them at random, the
+// others with an operand within 2^-28 of a power of two), nor any of the 2^18
+// reciprocals of the numbers below 2, which lie closest to halfway
 __device__ __forceinline__ double recip_nr(double b) {
   const double y = __builtin_amdgcn_rcp(b);
   const double e = fma(-b, y, 1.0);
@@ -71,14 +75,16 @@ __device__ __forceinline__ double inv_y(double b, double y) {
 // fixup handles zeros, infinities and NaN.  b is a product of (gamma - 1)
 // factors, so 0 or at least 2^-105 in magnitude; a is a sum of products of
 // pressures, zero or far above 2^-960, where the remainder would no longer be
-// exact.
+// exact.  Nor does a finite quotient overflow: it is an energy no larger than the
+// cells' that the pressure was reconstructed from (Kapila's squared sound speed,
+// a product of two pressures, overflows long before).
 __device__ __forceinline__ double div_const(double a, double b, double y) {
   return __builtin_amdgcn_div_fixup(div_y(a, b, y), b, a);
 }
 
-// sqrt(x) for x >= 2^-767, and for zero, infinity, NaN and negative x: one
-// coupled Newton step for the root g and its half reciprocal h (error below
-// 2^-44), then two corrections with the exact remainder x - g^2, the second of
+// sqrt(x) for x >= 2^-767, and for zero, infinity, NaN and negative x: one step of
+// Goldschmidt's coupled iteration for the root g and its half reciprocal h (error
+// below 2^-44), then two corrections with the exact remainder x - g^2, the second of
 // which rounds correctly.  Without the rescaling of tiny arguments it takes 13
 // instructions instead of 18.  Arguments are squared sound speeds, at least
 // 1e-12 or already reported as inadmissible.

@@ -74,8 +74,9 @@ int hype_strips(int nx) { return (nx + HYPE_TILE_W - 1) / HYPE_TILE_W; }
  * prologue).  Where the two halves of a tile run on two waves (pair), each
  * wave sweeps about h/2 rows plus one ring row, and the two meet at one
  * face (a quarter of an iteration).  Where they share every row (pair =
- * HYPE_LAYOUT_DUO), each takes about 0.54 of every row, ring rows included.  The
- * kernel is bound by FP64 issue:
+ * HYPE_LAYOUT_DUO), each takes about 0.54 of every row, ring rows included: the
+ * mean of the systems' shares, which is near enough to choose a height; duo_rows
+ * has each system's, to compare layouts with.  The kernel is bound by FP64 issue:
  * waves that share a SIMD share its issue slots, gaining only latency
  * hiding (a measured 1.5x for two waves).  With w = ceil(waves / simds)
  * waves per SIMD and `occ` resident waves per SIMD, a launch therefore takes
@@ -104,8 +105,10 @@ static double duo_rows(const hype_problem *p, int h)
     return share * (h + 2.0) + 1.0;
 }
 
-/* Time a wave takes for one row of a strip, in us: measured at order 2; order 3
- * takes about 1.3 times, orders 0 and 1 a third of that. */
+/* Time a wave takes for one row of a strip, in us: measured at order 2 with the
+ * kernels as duo_rows' shares were (those of today take some 5 % less, alike in
+ * all systems); order 3 takes about 1.3 times, orders 0 and 1 a third of that.
+ * Only the ratios matter (eng_auto_rows). */
 double hype_row_time(const hype_problem *p)
 {
     const double t = p->system == HYPE_EULER ? 4.87 : p->system == HYPE_KAPILA ? 9.0 : p->recons_prim ? 13.1 : 16.3;
